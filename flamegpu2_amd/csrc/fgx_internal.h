@@ -66,24 +66,27 @@ struct VarTable {
 
 int make_var_table(uint32_t nvars, const void* const* in, void* const* out, const uint32_t* bytes, VarTable* t);
 
+// Copy element `src_i` of variable `v` to element `dst_i` of its output array.
+__device__ __forceinline__ void copy_var(const VarTable& t, uint32_t v, uint32_t src_i, uint32_t dst_i) {
+    const uint32_t b = t.bytes[v];
+    const char* s = t.in[v] + (size_t)src_i * b;
+    char* d = t.out[v] + (size_t)dst_i * b;
+    if (b == 4) {
+        *reinterpret_cast<uint32_t*>(d) = *reinterpret_cast<const uint32_t*>(s);
+    } else if (b == 8) {
+        *reinterpret_cast<uint2*>(d) = *reinterpret_cast<const uint2*>(s);
+    } else if ((b & 3u) == 0) {
+        for (uint32_t w = 0; w < b; w += 4)
+            *reinterpret_cast<uint32_t*>(d + w) = *reinterpret_cast<const uint32_t*>(s + w);
+    } else {
+        for (uint32_t w = 0; w < b; ++w) d[w] = s[w];
+    }
+}
+
 // Copy element `src_i` of every variable (except `skip`) to element `dst_i` of its output array.
 __device__ __forceinline__ void copy_element(const VarTable& t, uint32_t src_i, uint32_t dst_i, int32_t skip = -1) {
-    for (uint32_t v = 0; v < t.n; ++v) {
-        if ((int32_t)v == skip) continue;
-        const uint32_t b = t.bytes[v];
-        const char* s = t.in[v] + (size_t)src_i * b;
-        char* d = t.out[v] + (size_t)dst_i * b;
-        if (b == 4) {
-            *reinterpret_cast<uint32_t*>(d) = *reinterpret_cast<const uint32_t*>(s);
-        } else if (b == 8) {
-            *reinterpret_cast<uint2*>(d) = *reinterpret_cast<const uint2*>(s);
-        } else if ((b & 3u) == 0) {
-            for (uint32_t w = 0; w < b; w += 4)
-                *reinterpret_cast<uint32_t*>(d + w) = *reinterpret_cast<const uint32_t*>(s + w);
-        } else {
-            for (uint32_t w = 0; w < b; ++w) d[w] = s[w];
-        }
-    }
+    for (uint32_t v = 0; v < t.n; ++v)
+        if ((int32_t)v != skip) copy_var(t, v, src_i, dst_i);
 }
 
 // Record dst_i of vt.rec from element src_i of the input variables (no-op without records).

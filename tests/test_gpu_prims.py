@@ -325,6 +325,41 @@ def test_pack_records(ctx, use_dn):
         fgx.pack_records(None, cap, ptr(d_w[0]), None, None, None, ptr(out) + 4)   # not 16-byte aligned
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 2047, 2049, 70_001])
+def test_compact_and_births_element_sizes(ctx, n):
+    # elements of every width side by side (pairs of 4-byte variables move together, 8-byte
+    # ones alone, others piecewise), the ID variable inside a pair, and births cut off by
+    # the list's capacity
+    from flamegpu2_amd import fgx
+    rng = np.random.default_rng(n)
+    flags = (rng.uniform(size=n) < 0.6).astype(np.uint32)
+    by = [4, 4, 8, 4, 12, 1, 2, 4, 4, 16]
+    raw = [rng.integers(0, 256, size=(n, b), dtype=np.uint8) for b in by]
+    d_f, d_in = dev(flags), [dev(r.reshape(-1)) for r in raw]
+    d_out = [empty(2 * n * b, np.uint8) for b in by]
+    d_cnt, d_nid, d_ovf = empty(1, np.uint32), dev(np.array([500], np.uint32)), empty(1, np.uint32)
+    sb = fgx.scratch_bytes(fgx.FGX_OP_COMPACT, n)
+    s = scratch(sb)
+    fgx.compact(ctx, ptr(d_f), 0, n, [ptr(t) for t in d_in], [ptr(t) for t in d_out], by, ptr(d_cnt), ptr(s), sb)
+    kept, born = np.nonzero(flags == 0)[0], np.nonzero(flags)[0]
+    cap = len(kept) + len(born) // 2
+    fgx.append_births(ctx, ptr(d_f), n, [ptr(t) for t in d_in], [ptr(t) for t in d_out], by, 8, ptr(d_cnt), cap,
+                      ptr(d_nid), ptr(s), sb, d_overflow=ptr(d_ovf))
+    sync()
+    assert int(host(d_cnt, np.uint32)[0]) == cap
+    assert int(host(d_ovf, np.uint32)[0]) == (1 if len(born) > len(born) // 2 else 0)
+    assert int(host(d_nid, np.uint32)[0]) == 500 + len(born)
+    at = np.concatenate([kept, born])[:cap]
+    for v, b in enumerate(by):
+        got = host(d_out[v], np.uint8, 2 * n * b).reshape(2 * n, b)
+        exp = raw[v][at]
+        if v == 8:
+            exp = exp.copy()
+            exp[len(kept):] = (500 + np.arange(cap - len(kept), dtype=np.uint32)).view(np.uint8).reshape(-1, 4)
+        assert np.array_equal(got[:cap], exp), f"variable {v} ({b} bytes)"
+        assert not got[cap:].any()
+
+
 def test_compact_device_count(ctx):
     from flamegpu2_amd import fgx
     rng = np.random.default_rng(3)
