@@ -352,7 +352,7 @@ int fgx_reduce_sum(fgx_ctx* ctx, int type, const void* in, const uint32_t* d_n, 
  *   [0] sum, [1] min, [2] max  as double (f32/f64), int64 (i32/i64) or uint64 (u32/u64);
  *   [3] sum over items of ((double)x - sum / n)^2 as double (0 when n == 0).
  * min/max of an empty list are the type's largest / lowest value (the reduction identities).
- * Deterministic: a fixed-shape tree, so the bits do not depend on scheduling.  Four
+ * Deterministic: a fixed-shape tree, so the bits do not depend on scheduling.  Two
  * launches, no host synchronisation.  Scratch: fgx_scratch_bytes(FGX_OP_STATS, 0, 0). */
 int fgx_reduce_stats(fgx_ctx* ctx, int type, const void* in, const uint32_t* d_n, uint32_t n_cap,
                      void* d_out, void* scratch, size_t scratch_bytes, void* stream);

@@ -637,3 +637,24 @@ def test_reduce_stats(ctx, code, dtype, acc, n):
     d = a.astype(np.float64) - mean
     ref = float((d * d).sum())
     assert abs(sq - ref) <= 1e-10 * max(ref, 1.0)
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 200 * 1024, 200 * 1024 + 1, 8 * 200 * 1024 - 1, 8 * 200 * 1024 + 3])
+def test_reduce_stats_block_edges(ctx, n):
+    # sizes around the blocks and batches of the one-pass statistics, on values far from zero
+    # and close together, where squared deviations are the digits that a sum of squares loses.
+    # Bound: the deviations are exact to a few units in the last place of a double each
+    # (2^-53), and merging at most 64 sets adds as many roundings: 1e-13 leaves a factor of ten
+    from flamegpu2_amd import fgx
+    a = (1.0e6 + np.random.default_rng(n).normal(size=n)).astype(np.float64)
+    sb = fgx.scratch_bytes(fgx.FGX_OP_STATS, 0)
+    s = scratch(sb)
+    o = empty(4, np.float64)
+    fgx.reduce_stats(ctx, 1, ptr(dev(a)), n, ptr(o), ptr(s), sb)
+    sync()
+    sm, mn, mx, sq = host(o, np.float64, 4)
+    x = a.astype(np.longdouble)
+    ref = ((x - x.mean()) ** 2).sum()
+    assert mn == a.min() and mx == a.max()
+    assert abs(sm - float(x.sum())) <= 1e-13 * float(x.sum())
+    assert abs(sq - float(ref)) <= 1e-13 * float(ref) + 1e-300
