@@ -36,7 +36,7 @@ HIP_FLAGS = [
 ]
 
 # target name -> (sources, link libs)
-LIBFGX_SRCS = ["fgx_core.hip", "fgx_prims.hip"]
+LIBFGX_SRCS = ["fgx_core.hip", "fgx_prims.hip", "fgx_bucket_sort.hip"]
 
 
 def _run(cmd):

@@ -1,0 +1,770 @@
+// Stable sort of a list's elements by bin, through LDS, for gfx950 (wave64).
+//
+//   count   per tile of the list: how many elements fall into each bucket of bins
+//   prefix  per bucket: the elements of the tiles before
+//   split   per tile: (bin within the bucket, element index) to the bucket, stably
+//   sort    per bucket: stable order by bin in LDS, the bin starts, and every variable
+//
+// Ranks are taken in list order (per-wave counters, and the lanes of a wave that share a
+// key), so no pass depends on the order in which atomics land and none has to restore it.
+// Lists of one tile are sorted by one block in one launch.
+//
+// What bounds it: from some 100,000 elements on, the gathers and stores of the last pass;
+// below, the launches, of which there are four (the sort through global atomics takes
+// seven).  1,048,576 messages of 28 bytes over 64^3 bins, in the order of the step before:
+// 69.3 us with atomics, 52.1 us this way; 8,388,593 of 20 bytes in no order: 2,069 and 528 us;
+// sort of 250,007 agents: 36.4 and 31.2 us.
+#include "fgx_bucket_sort.h"
+
+#include <algorithm>
+
+namespace fgx {
+
+constexpr uint32_t kMaxBuckets = 2048;     // per-wave 16-bit counters of a split: 64 KB for 16 waves
+
+struct BucketArgs {
+    KeyArgs ka;
+    const uint32_t* d_n;
+    uint32_t n_cap;
+    uint32_t shift, buckets, tiles, bins;
+    const float* x;
+    const float* y;
+    const float* z;
+    uint32_t* counts;     // [tiles][buckets] elements; after the prefix pass those of the tiles before
+    uint32_t* totals;     // [buckets] elements
+    uint32_t* starts;     // [buckets + 1] first element
+    uint32_t* met;        // [tiles] buckets that occur in the tile
+    uint32_t* stage;      // one word: the split moves the variables too (see k_bucket_split)
+    uint32_t stage_above; // sum of `met` above which it does; 0: never
+    uint16_t* fine;       // bin within the bucket, in bucket order
+    uint32_t* idx;        // element index, in bucket order
+    uint32_t* start_out;  // bin starts, or NULL
+};
+
+__device__ __forceinline__ uint32_t key_of(const BucketArgs& a, uint32_t i) {
+    return bin_key(a.ka, a.x[i], a.y[i], a.ka.dims == 3 ? a.z[i] : 0.0f);
+}
+
+// Exclusive sum over the block's threads (W waves); *total receives the block's sum.
+template <uint32_t W>
+__device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* s_red, uint32_t* total) {
+    const uint32_t w = threadIdx.x >> 6;
+    const uint32_t incl = wave_inclusive_u32(v);
+    __syncthreads();   // s_red may still be read by the call before
+    if (lane_id() == 63) s_red[w] = incl;
+    __syncthreads();
+    uint32_t off = 0, tot = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < W; ++k) {
+        off += k < w ? s_red[k] : 0u;
+        tot += s_red[k];
+    }
+    *total = tot;
+    return off + incl - v;
+}
+
+// ---------------------------------------------------------------- stable split in LDS
+// Elements are numbered (wave, chunk, lane); rows[w * keys + k] counts wave w's elements of
+// key k in 16 bits (a wave holds at most 1,024).
+__device__ __forceinline__ void split_count(uint16_t* rows, uint32_t row, uint32_t k) {
+    const uint32_t at = row + k;
+    atomicAdd(reinterpret_cast<uint32_t*>(rows) + (at >> 1), 1u << ((at & 1u) * 16u));
+}
+
+// After the counts: rows become each wave's first place within its key, s_start the keys'
+// first places.  Thread t owns keys [t * q, t * q + q).
+template <uint32_t W>
+__device__ __forceinline__ void split_scan(uint16_t* rows, uint32_t stride, uint32_t keys, uint32_t* s_start,
+                                           uint32_t* s_red) {
+    const uint32_t q = (keys + W * 64u - 1u) / (W * 64u);
+    const uint32_t k0 = threadIdx.x * q;
+    uint32_t sum = 0;
+    for (uint32_t j = 0; j < q && k0 + j < keys; ++j) {
+        uint32_t c[W];
+#pragma unroll
+        for (uint32_t w = 0; w < W; ++w) c[w] = rows[w * stride + k0 + j];
+        uint32_t run = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < W; ++w) {
+            rows[w * stride + k0 + j] = (uint16_t)run;
+            run += c[w];
+        }
+        s_start[k0 + j] = run;
+        sum += run;
+    }
+    uint32_t total;
+    uint32_t base = block_prefix<W>(sum, s_red, &total);
+    for (uint32_t j = 0; j < q && k0 + j < keys; ++j) {
+        const uint32_t c = s_start[k0 + j];
+        s_start[k0 + j] = base;
+        base += c;
+    }
+    __syncthreads();
+}
+
+// The place of one element of the wave's next chunk.  Lanes with the same key take places in
+// lane order; the last of them moves the wave's counter on (LDS runs a wave's accesses in
+// program order, which `volatile` keeps).
+__device__ __forceinline__ uint32_t split_place(uint16_t* s_rows, const uint32_t* s_start, uint32_t row, uint32_t k,
+                                                bool valid, uint32_t bits) {
+    volatile __attribute__((address_space(3))) uint16_t* rows = (__attribute__((address_space(3))) uint16_t*)s_rows;
+    uint64_t same = __ballot(valid);
+    for (uint32_t b = 0; b < bits; ++b) {
+        const bool on = (k >> b) & 1u;
+        const uint64_t m = __ballot(on);
+        same &= on ? m : ~m;
+    }
+    if (!valid) return 0u;
+    const uint32_t lane = lane_id();
+    const uint32_t before = rows[row + k];
+    const uint32_t place = s_start[k] + before + (uint32_t)__builtin_popcountll(same & ((1ull << lane) - 1ull));
+    if (lane == 63u - (uint32_t)__builtin_clzll(same)) rows[row + k] = (uint16_t)(before + (uint32_t)__builtin_popcountll(same));
+    return place;
+}
+
+__device__ __forceinline__ uint32_t key_bits(uint32_t keys) { return keys > 1u ? 32u - (uint32_t)__builtin_clz(keys - 1u) : 0u; }
+
+template <uint32_t BT>
+__device__ __forceinline__ void zero_rows(uint16_t* rows, uint32_t n) {
+    for (uint32_t k = threadIdx.x; k < (n + 1u) / 2u; k += BT) reinterpret_cast<uint32_t*>(rows)[k] = 0u;
+}
+
+// ---------------------------------------------------------------- count
+template <uint32_t BT, uint32_t ITEMS>
+__global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
+    __shared__ uint32_t s_hist[kMaxBuckets];
+    __shared__ uint32_t s_met;
+    const uint32_t tile = xcd_block(), t = threadIdx.x;
+    const uint32_t n = load_count(a.d_n, a.n_cap);
+    for (uint32_t b = t; b < a.buckets; b += BT) s_hist[b] = 0u;
+    if (t == 0) s_met = 0u;
+    __syncthreads();
+    const uint32_t base = tile * BT * ITEMS;
+    if (base < n) {
+        uint32_t k[ITEMS];
+#pragma unroll
+        for (uint32_t j = 0; j < ITEMS; ++j) {
+            const uint32_t i = base + j * BT + t;
+            k[j] = key_of(a, i < n ? i : base) >> a.shift;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < ITEMS; ++j)
+            if (base + j * BT + t < n) atomicAdd(&s_hist[k[j]], 1u);
+    }
+    __syncthreads();
+    uint32_t met = 0;
+    for (uint32_t b = t; b < a.buckets; b += BT) {
+        const uint32_t c = s_hist[b];
+        a.counts[(size_t)tile * a.buckets + b] = c;
+        met += c ? 1u : 0u;
+    }
+    if (!a.stage_above) return;
+    met = wave_sum_u32(met);
+    if (lane_id() == 0) atomicAdd(&s_met, met);
+    __syncthreads();
+    if (t == 0) a.met[tile] = s_met;
+}
+
+// ---------------------------------------------------------------- prefix
+// Block g: buckets [64 g, 64 g + 64), one per lane; each of the 16 waves takes a run of the
+// tiles, 8 loads in flight.
+__global__ void __launch_bounds__(1024) k_bucket_prefix(BucketArgs a) {
+    __shared__ uint32_t s_sum[16][64];
+    __shared__ uint32_t s_red[16];
+    const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
+    const uint32_t b = blockIdx.x * 64u + lane;
+    const uint32_t per = (a.tiles + 15u) / 16u;
+    const uint32_t t0 = w * per < a.tiles ? w * per : a.tiles, t1 = t0 + per < a.tiles ? t0 + per : a.tiles;
+    const bool on = b < a.buckets;
+    uint32_t sum = 0;
+    for (uint32_t t = t0; t < t1; t += 8u) {
+        uint32_t c[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) c[j] = on && t + j < t1 ? a.counts[(size_t)(t + j) * a.buckets + b] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) sum += c[j];
+    }
+    s_sum[w][lane] = sum;
+    __syncthreads();
+    uint32_t run = 0, total = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k) {
+        run += k < w ? s_sum[k][lane] : 0u;
+        total += s_sum[k][lane];
+    }
+    for (uint32_t t = t0; t < t1; t += 8u) {
+        uint32_t c[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) c[j] = on && t + j < t1 ? a.counts[(size_t)(t + j) * a.buckets + b] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            if (on && t + j < t1) a.counts[(size_t)(t + j) * a.buckets + b] = run;
+            run += c[j];
+        }
+    }
+    if (w == 0 && on) a.totals[b] = total;
+    if (blockIdx.x == 0) {
+        uint32_t met = 0, all = 0;
+        if (a.stage_above)
+            for (uint32_t t = threadIdx.x; t < a.tiles; t += 1024u) met += a.met[t];
+        block_prefix<16>(met, s_red, &all);
+        if (threadIdx.x == 0) *a.stage = a.stage_above && all > a.stage_above ? 1u : 0u;
+    }
+}
+
+// ---------------------------------------------------------------- split
+// A tile's elements in bucket order are laid out in LDS first, so that the stores to each
+// bucket are runs.  When the list is in no order (a tile meets so many buckets that its
+// elements of one are fewer than a cache line's worth), the variables move with the split,
+// to the bucket's place in the output arrays: the last pass then permutes each bucket in
+// place, where it would otherwise gather every element's line of every variable from the
+// whole list.
+template <uint32_t BT, uint32_t ITEMS, uint32_t MAXB>
+__global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) {
+    constexpr uint32_t W = BT / 64u, T = BT * ITEMS;
+    __shared__ alignas(16) uint16_t s_rows[W * MAXB];
+    __shared__ uint32_t s_start[MAXB];
+    __shared__ uint32_t s_delta[MAXB];
+    __shared__ uint32_t s_key[T];
+    __shared__ uint16_t s_loc[T];
+    __shared__ uint32_t s_red[W];
+    const uint32_t tile = xcd_block(), t = threadIdx.x, w = t >> 6, lane = lane_id();
+    const uint32_t n = load_count(a.d_n, a.n_cap), nb = a.buckets;
+    const uint32_t base = tile * T;
+    if (base >= n && tile != 0) return;
+    const uint32_t cnt = base < n ? (n - base < T ? n - base : T) : 0u;
+    // this thread's buckets: their totals and the tile's offsets are loaded beside the positions
+    constexpr uint32_t Q = MAXB / BT;
+    const uint32_t q = (nb + BT - 1u) / BT, b0 = t * q;
+    uint32_t total_of[Q], offset_of[Q];
+#pragma unroll
+    for (uint32_t j = 0; j < Q; ++j) {
+        const bool on = j < q && b0 + j < nb;
+        total_of[j] = on ? a.totals[b0 + j] : 0u;
+        offset_of[j] = on ? a.counts[(size_t)tile * nb + b0 + j] : 0u;
+    }
+    uint32_t key[ITEMS];
+#pragma unroll
+    for (uint32_t c = 0; c < ITEMS; ++c) {
+        const uint32_t e = (w * ITEMS + c) * 64u + lane;
+        key[c] = cnt ? key_of(a, base + (e < cnt ? e : 0u)) : 0u;
+    }
+    zero_rows<BT>(s_rows, W * nb);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t c = 0; c < ITEMS; ++c)
+        if ((w * ITEMS + c) * 64u + lane < cnt) split_count(s_rows, w * nb, key[c] >> a.shift);
+    __syncthreads();
+    split_scan<W>(s_rows, nb, nb, s_start, s_red);
+    // where the tile's elements of each bucket go: the bucket's start + those of the tiles before
+    {
+        uint32_t sum = 0, total;
+#pragma unroll
+        for (uint32_t j = 0; j < Q; ++j) sum += total_of[j];
+        uint32_t run = block_prefix<W>(sum, s_red, &total);
+#pragma unroll
+        for (uint32_t j = 0; j < Q; ++j) {
+            if (j >= q || b0 + j >= nb) continue;
+            s_delta[b0 + j] = run + offset_of[j] - s_start[b0 + j];
+            if (tile == 0) a.starts[b0 + j] = run;
+            run += total_of[j];
+        }
+        if (tile == 0 && t == 0) a.starts[nb] = total;
+    }
+    const uint32_t bits = key_bits(nb);
+#pragma unroll
+    for (uint32_t c = 0; c < ITEMS; ++c) {
+        const uint32_t e = (w * ITEMS + c) * 64u + lane;
+        const bool valid = e < cnt;
+        const uint32_t p = split_place(s_rows, s_start, w * nb, key[c] >> a.shift, valid, bits);
+        if (valid) {
+            s_key[p] = key[c];
+            s_loc[p] = (uint16_t)e;
+        }
+    }
+    __syncthreads();
+    const uint32_t mask = (1u << a.shift) - 1u;
+    uint32_t src[ITEMS], dst[ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < ITEMS; ++j) {
+        const uint32_t p = j * BT + t;
+        src[j] = dst[j] = 0u;
+        if (p < cnt) {
+            const uint32_t k = s_key[p];
+            dst[j] = s_delta[k >> a.shift] + p;
+            src[j] = base + s_loc[p];
+            a.fine[dst[j]] = (uint16_t)(k & mask);
+            a.idx[dst[j]] = src[j];
+        }
+    }
+    if (!*a.stage) return;
+    for (uint32_t v = 0; v < vt.n; ++v) {
+        if (vt.bytes[v] == 4) {
+            const uint32_t* in = reinterpret_cast<const uint32_t*>(vt.in[v]);
+            uint32_t* out = reinterpret_cast<uint32_t*>(vt.out[v]);
+            uint32_t x[ITEMS];
+#pragma unroll
+            for (uint32_t j = 0; j < ITEMS; ++j)
+                if (j * BT + t < cnt) x[j] = in[src[j]];
+#pragma unroll
+            for (uint32_t j = 0; j < ITEMS; ++j)
+                if (j * BT + t < cnt) out[dst[j]] = x[j];
+        } else {
+            for (uint32_t j = 0; j < ITEMS; ++j)
+                if (j * BT + t < cnt) copy_var(vt, v, src[j], dst[j]);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- sort within a bucket
+// Writes output elements first + [0, m): place p takes input element s_src[p] (or in[first + p]
+// when s_src is NULL).  Two places and up to eight 4-byte variables per thread are loaded
+// before the first store.
+template <uint32_t BT>
+__device__ __forceinline__ void write_sorted(const VarTable& vt, const uint32_t* s_src, const uint32_t* in, uint32_t first,
+                                             uint32_t m) {
+    constexpr uint32_t P = 2, V = 8;
+    for (uint32_t p0 = threadIdx.x; p0 < m; p0 += P * BT) {
+        uint32_t e[P];
+        bool on[P];
+#pragma unroll
+        for (uint32_t j = 0; j < P; ++j) {
+            const uint32_t p = p0 + j * BT;
+            on[j] = p < m;
+            e[j] = on[j] ? (s_src ? s_src[p] : in[first + p]) : 0u;
+        }
+        uint32_t r[4][P] = {};
+        for (uint32_t v0 = 0; v0 < vt.n; v0 += V) {
+            uint32_t x[V][P];
+#pragma unroll
+            for (uint32_t k = 0; k < V; ++k) {
+                if (v0 + k >= vt.n || vt.bytes[v0 + k] != 4) continue;
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(vt.in[v0 + k]);
+#pragma unroll
+                for (uint32_t j = 0; j < P; ++j)
+                    if (on[j]) x[k][j] = src[e[j]];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < V; ++k) {
+                if (v0 + k >= vt.n) continue;
+                if (vt.bytes[v0 + k] == 4) {
+                    uint32_t* out = reinterpret_cast<uint32_t*>(vt.out[v0 + k]);
+#pragma unroll
+                    for (uint32_t j = 0; j < P; ++j)
+                        if (on[j]) out[first + p0 + j * BT] = x[k][j];
+                    // the record's words are variables just loaded (a second gather of four words
+                    // cost as much as four variables: 29.1 against 23.5 us for 1 M messages)
+#pragma unroll
+                    for (uint32_t c = 0; c < 4; ++c) {
+                        if (vt.rec_var[c] != (int32_t)(v0 + k)) continue;
+#pragma unroll
+                        for (uint32_t j = 0; j < P; ++j) r[c][j] = x[k][j];
+                    }
+                } else {
+                    for (uint32_t j = 0; j < P; ++j)
+                        if (on[j]) copy_var(vt, v0 + k, e[j], first + p0 + j * BT);
+                }
+            }
+        }
+        if (vt.rec) {
+#pragma unroll
+            for (uint32_t j = 0; j < P; ++j)
+                if (on[j]) reinterpret_cast<uint4*>(vt.rec)[first + p0 + j * BT] = make_uint4(r[0][j], r[1][j], r[2][j], r[3][j]);
+        }
+    }
+}
+
+// The same for a bucket whose variables the split has moved to the output arrays already: place
+// p takes element first + s_src[p] of the output arrays, so all of a variable's m <= S * BT
+// elements are read before the first of them is written.
+template <uint32_t BT, uint32_t S>
+__device__ __forceinline__ void permute_sorted(const VarTable& vt, const uint32_t* s_src, uint32_t first, uint32_t m) {
+    const uint32_t t = threadIdx.x;
+    uint32_t e[S];
+#pragma unroll
+    for (uint32_t j = 0; j < S; ++j) e[j] = first + (j * BT + t < m ? s_src[j * BT + t] : 0u);
+    if (vt.rec) {
+#pragma unroll
+        for (uint32_t j0 = 0; j0 < S; j0 += 2) {
+            uint32_t r[4][2];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const int32_t v = vt.rec_var[k];
+#pragma unroll
+                for (uint32_t j = 0; j < 2; ++j)
+                    r[k][j] = v >= 0 && (j0 + j) * BT + t < m
+                                  ? reinterpret_cast<const uint32_t*>(vt.out[v < 0 ? 0 : v])[e[j0 + j]] : 0u;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j)
+                if ((j0 + j) * BT + t < m)
+                    reinterpret_cast<uint4*>(vt.rec)[first + (j0 + j) * BT + t] = make_uint4(r[0][j], r[1][j], r[2][j], r[3][j]);
+        }
+        __syncthreads();   // the records are read from arrays that are permuted next
+    }
+    for (uint32_t v = 0; v < vt.n; ++v) {
+        // elements of any size move as words, or as bytes: piece by piece, each of them read by
+        // every thread before any is written
+        const uint32_t b = vt.bytes[v], step = (b & 3u) ? 1u : 4u;
+        for (uint32_t at = 0; at < b; at += step) {
+            uint32_t x[S];
+#pragma unroll
+            for (uint32_t j = 0; j < S; ++j) {
+                x[j] = 0u;
+                if (j * BT + t >= m) continue;
+                const char* s = vt.out[v] + (size_t)e[j] * b + at;
+                x[j] = step == 4 ? *reinterpret_cast<const uint32_t*>(s) : (uint32_t)*reinterpret_cast<const uint8_t*>(s);
+            }
+            // every load is back before any thread stores: the loaded values are used here
+#pragma unroll
+            for (uint32_t j = 0; j < S; ++j) asm volatile("" ::"v"(x[j]));
+            __syncthreads();
+#pragma unroll
+            for (uint32_t j = 0; j < S; ++j) {
+                if (j * BT + t >= m) continue;
+                char* d = vt.out[v] + (size_t)(first + j * BT + t) * b + at;
+                if (step == 4) *reinterpret_cast<uint32_t*>(d) = x[j];
+                else *reinterpret_cast<uint8_t*>(d) = (uint8_t)x[j];
+            }
+        }
+    }
+}
+
+// LDS of one sorting block: the split's counters, and in the same words (before they are
+// counted) the bins of a selected part of an oversize bucket; the sources of each place.
+template <uint32_t BT, uint32_t MAXF, uint32_t S>
+struct SortLds {
+    static constexpr uint32_t kCap = BT * S;   // S elements per thread
+    static constexpr uint32_t kRowWords = (BT / 64u) * MAXF / 2u;
+    uint32_t rows[kRowWords > kCap / 2u ? kRowWords : kCap / 2u];
+    uint32_t start[MAXF + 1];
+    uint32_t src[kCap];
+    uint32_t red[BT / 64u];
+    uint32_t lo, hi;
+};
+
+// Elements (f[c], id[c]) of chunk c < cw of each wave, m in all, numbered (wave, chunk, lane):
+// s.src[place] = id in stable order by f, s.start[f] = first place.
+template <uint32_t BT, uint32_t MAXF, uint32_t S>
+__device__ __forceinline__ void sort_in_lds(SortLds<BT, MAXF, S>& s, uint32_t keys, const uint32_t (&f)[S],
+                                            const uint32_t (&id)[S], uint32_t cw, uint32_t m) {
+    constexpr uint32_t W = BT / 64u;
+    const uint32_t w = threadIdx.x >> 6, lane = lane_id();
+    uint16_t* rows = reinterpret_cast<uint16_t*>(s.rows);
+    const uint32_t stride = (keys + 1u) & ~1u;
+    zero_rows<BT>(rows, W * stride);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t c = 0; c < S; ++c)
+        if (c < cw && (w * cw + c) * 64u + lane < m) split_count(rows, w * stride, f[c]);
+    __syncthreads();
+    split_scan<W>(rows, stride, keys, s.start, s.red);
+    const uint32_t bits = key_bits(keys);
+#pragma unroll
+    for (uint32_t c = 0; c < S; ++c) {
+        if (c >= cw) continue;
+        const bool valid = (w * cw + c) * 64u + lane < m;
+        const uint32_t p = split_place(rows, s.start, w * stride, f[c], valid, bits);
+        if (valid) s.src[p] = id[c];
+    }
+    __syncthreads();
+}
+
+// A bucket of more elements than its block holds is shared by several blocks: block `piece`
+// orders the bins that start within its window of kCap / 2 places.  The bucket's bins are
+// counted, the bins of the window selected in order into LDS, and sorted there; a bin that is
+// larger than LDS is already in order and is written as it comes.
+template <uint32_t BT, uint32_t MAXF, uint32_t S>
+__device__ __forceinline__ void sort_piece(const BucketArgs& a, const VarTable& vt, SortLds<BT, MAXF, S>& s, uint32_t bucket, uint32_t first,
+                           uint32_t m, uint32_t piece, uint32_t pieces) {
+    constexpr uint32_t W = BT / 64u, kCap = SortLds<BT, MAXF, S>::kCap, kWindow = kCap / 2u;
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
+    const uint32_t keys = 1u << a.shift;
+    for (uint32_t k = t; k < keys; k += BT) s.start[k] = 0u;
+    if (t == 0) {
+        s.lo = 0xFFFFFFFFu;
+        s.hi = 0u;
+    }
+    __syncthreads();
+    for (uint32_t e = t; e < m; e += BT) atomicAdd(&s.start[a.fine[first + e]], 1u);
+    __syncthreads();
+    {
+        const uint32_t q = (keys + BT - 1u) / BT, k0 = t * q;
+        uint32_t sum = 0, total;
+        for (uint32_t j = 0; j < q && k0 + j < keys; ++j) sum += s.start[k0 + j];
+        uint32_t run = block_prefix<W>(sum, s.red, &total);
+        const uint32_t lo = piece * kWindow, hi = piece + 1u == pieces ? 0xFFFFFFFFu : lo + kWindow;
+        for (uint32_t j = 0; j < q && k0 + j < keys; ++j) {
+            const uint32_t k = k0 + j, c = s.start[k];
+            s.start[k] = run;
+            if (run >= lo && run < hi) {
+                atomicMin(&s.lo, k);
+                if (c) atomicMax(&s.hi, k + 1u);
+                const uint32_t bin = (bucket << a.shift) + k;
+                if (a.start_out && bin < a.bins) a.start_out[bin] = first + run;
+            }
+            run += c;
+        }
+        if (t == 0) s.start[keys] = m;
+    }
+    __syncthreads();
+    const uint32_t ka = s.lo, kb = s.hi;     // bins [ka, kb) hold the window's elements
+    if (ka >= kb) return;
+    const uint32_t p0 = s.start[ka], p1 = s.start[kb];
+    uint32_t kc = kb;                        // bins [ka, kc) are sorted in LDS
+    if (p1 - p0 > kCap) kc = kb - 1u;        // the last one is too large (all before it start within the window)
+    const uint32_t pc = s.start[kc];
+    __syncthreads();
+    uint32_t taken = 0, passed = 0;
+    uint16_t* s_fine = reinterpret_cast<uint16_t*>(s.rows);
+    for (uint32_t e0 = 0; e0 < m; e0 += BT) {
+        const uint32_t e = e0 + t;
+        const uint32_t f = e < m ? a.fine[first + e] : 0xFFFFFFFFu;
+        const bool sel = f >= ka && f < kc, big = f >= kc && f < kb;
+        const uint64_t ms = __ballot(sel), mb = __ballot(big);
+        __syncthreads();
+        if (lane == 0) s.red[w] = (uint32_t)__builtin_popcountll(ms) | (uint32_t)__builtin_popcountll(mb) << 16;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < W; ++k) {
+            before += k < w ? s.red[k] : 0u;
+            all += s.red[k];
+        }
+        const uint64_t below = (1ull << lane) - 1ull;
+        if (sel) {
+            const uint32_t p = taken + (before & 0xFFFFu) + (uint32_t)__builtin_popcountll(ms & below);
+            s_fine[p] = (uint16_t)(f - ka);
+            s.src[p] = a.idx[first + e];
+        }
+        if (big) {
+            const uint32_t p = first + pc + passed + (before >> 16) + (uint32_t)__builtin_popcountll(mb & below);
+            const uint32_t i = a.idx[first + e];
+            copy_element(vt, i, p);
+            write_record(vt, i, p);
+        }
+        taken += all & 0xFFFFu;
+        passed += all >> 16;
+    }
+    __syncthreads();
+    if (!taken) return;
+    const uint32_t cw = ((taken + 63u) / 64u + W - 1u) / W;
+    uint32_t f[S], id[S];
+#pragma unroll
+    for (uint32_t c = 0; c < S; ++c) {
+        const uint32_t e = (w * cw + c) * 64u + lane;
+        const bool valid = c < cw && e < taken;
+        f[c] = valid ? s_fine[e] : 0u;
+        id[c] = valid ? s.src[e] : 0u;
+    }
+    __syncthreads();
+    sort_in_lds<BT, MAXF, S>(s, kc - ka, f, id, cw, taken);
+    write_sorted<BT>(vt, s.src, nullptr, first + p0, taken);
+}
+
+// Two blocks of 1,024 threads share a CU where S is 8 (at most 64 VGPRs): one loads while the
+// other ranks.
+template <uint32_t BT, uint32_t MAXF, uint32_t S>
+__global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a, VarTable vt) {
+    constexpr uint32_t W = BT / 64u, kCap = SortLds<BT, MAXF, S>::kCap, kWindow = kCap / 2u;
+    __shared__ SortLds<BT, MAXF, S> s;
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id(), nb = a.buckets;
+    uint32_t b, piece = 0;
+    if (blockIdx.x < nb) {
+        // one block per bucket, neighbouring buckets on one XCD
+        const uint32_t x = blockIdx.x % 8u, k = blockIdx.x / 8u, q = nb / 8u, r = nb % 8u;
+        b = x * q + (x < r ? x : r) + k;
+    } else {
+        // further blocks: the pieces after the first of buckets that one block does not hold
+        const uint32_t q = (nb + BT - 1u) / BT, b0 = t * q, want = blockIdx.x - nb;
+        if (t == 0) s.lo = 0xFFFFFFFFu;
+        uint32_t sum = 0, total;
+        for (uint32_t j = 0; j < q && b0 + j < nb; ++j) {
+            const uint32_t m = a.starts[b0 + j + 1u] - a.starts[b0 + j];
+            sum += m > kCap ? (m - 1u) / kWindow : 0u;
+        }
+        uint32_t run = block_prefix<W>(sum, s.red, &total);
+        if (want >= total) return;
+        for (uint32_t j = 0; j < q && b0 + j < nb; ++j) {
+            const uint32_t m = a.starts[b0 + j + 1u] - a.starts[b0 + j];
+            const uint32_t more = m > kCap ? (m - 1u) / kWindow : 0u;
+            if (want >= run && want < run + more) {
+                s.lo = b0 + j;
+                s.hi = want - run + 1u;
+            }
+            run += more;
+        }
+        __syncthreads();
+        b = s.lo;
+        piece = s.hi;
+        __syncthreads();
+    }
+    const uint32_t first = a.starts[b], m = a.starts[b + 1u] - first;
+    if (a.start_out && b == nb - 1u && piece == 0 && t == 0) a.start_out[a.bins] = first + m;
+    if (a.shift == 0) {
+        // a bucket is one bin and already in order
+        if (a.start_out && piece == 0 && t == 0) a.start_out[b] = first;
+        const uint32_t p = m > kCap ? piece * kWindow : 0u;
+        const uint32_t len = m > kCap ? (m - p < kWindow ? m - p : kWindow) : m;
+        write_sorted<BT>(vt, nullptr, a.idx, first + p, len);
+        return;
+    }
+    if (m == 0) {
+        if (a.start_out)
+            for (uint32_t k = t; k < 1u << a.shift; k += BT)
+                if ((b << a.shift) + k < a.bins) a.start_out[(b << a.shift) + k] = first;
+        return;
+    }
+    if (m > kCap) {
+        sort_piece<BT, MAXF, S>(a, vt, s, b, first, m, piece, (m - 1u) / kWindow + 1u);
+        return;
+    }
+    const bool staged = *a.stage != 0u;
+    const uint32_t cw = ((m + 63u) / 64u + W - 1u) / W;
+    uint32_t f[S], id[S];
+#pragma unroll
+    for (uint32_t c = 0; c < S; ++c) {
+        const uint32_t e = (w * cw + c) * 64u + lane;
+        const bool valid = c < cw && e < m;
+        f[c] = valid ? a.fine[first + e] : 0u;
+        id[c] = staged ? e : (valid ? a.idx[first + e] : 0u);
+    }
+    const uint32_t keys = 1u << a.shift;
+    sort_in_lds<BT, MAXF, S>(s, keys, f, id, cw, m);
+    if (a.start_out)
+        for (uint32_t k = t; k < keys; k += BT)
+            if ((b << a.shift) + k < a.bins) a.start_out[(b << a.shift) + k] = first + s.start[k];
+    if (staged) permute_sorted<BT, S>(vt, s.src, first, m);
+    else write_sorted<BT>(vt, s.src, nullptr, first, m);
+}
+
+// The whole list by one block: keys from the positions, sorted in LDS.
+template <uint32_t BT, uint32_t MAXF, uint32_t S>
+__global__ void __launch_bounds__(BT) k_sort_one_block(BucketArgs a, VarTable vt) {
+    constexpr uint32_t W = BT / 64u;
+    __shared__ SortLds<BT, MAXF, S> s;
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
+    const uint32_t n = load_count(a.d_n, a.n_cap);
+    const uint32_t cw = ((n + 63u) / 64u + W - 1u) / W;
+    uint32_t f[S], id[S];
+#pragma unroll
+    for (uint32_t c = 0; c < S; ++c) {
+        const uint32_t e = (w * cw + c) * 64u + lane;
+        const bool valid = c < cw && e < n;
+        f[c] = valid ? key_of(a, e) : 0u;
+        id[c] = e;
+    }
+    sort_in_lds<BT, MAXF, S>(s, a.bins, f, id, cw, n);
+    if (a.start_out) {
+        for (uint32_t k = t; k < a.bins; k += BT) a.start_out[k] = s.start[k];
+        if (t == 0) a.start_out[a.bins] = n;
+    }
+    write_sorted<BT>(vt, s.src, nullptr, 0u, n);
+}
+
+// ---------------------------------------------------------------- host
+constexpr uint32_t kOneBlockMax = 4096u;
+constexpr uint32_t kMaxBins = 1024u;       // bins of a bucket: a sorting block's counters
+
+bool bucket_plan(uint32_t n_cap, uint32_t bins, uint64_t used, BucketPlan* p) {
+    // beyond 12 M elements the buckets outgrow their blocks
+    if (!n_cap || !bins || n_cap > (3u << 22)) return false;
+    *p = BucketPlan{};
+    // one block sorts a list of 1,024 elements in 7 us; the four passes take 23 us on one of
+    // 16,384, launches and all
+    if (n_cap <= kOneBlockMax && bins <= kMaxBins) {
+        p->one_block = 1;
+        p->threads = 1024;
+        return true;
+    }
+    // Elements per bucket, at most (the bins that occur evenly filled): a half or less of what
+    // a sorting block holds, so that denser regions still fit.  Lists below 262,144 elements
+    // take blocks of 256 threads (2,048 elements), and smaller buckets below 65,536, so that
+    // there are enough blocks; larger ones 1,024 threads (8,192 elements); from 3 M on the
+    // buckets a tile can count are too few for that (16,384 elements, tiles of 8,192).
+    uint32_t per, most;
+    if (n_cap < (1u << 18)) {
+        p->threads = 256;
+        p->items = 4;
+        per = n_cap < (1u << 16) ? 256 : 1024;
+        most = 1024;
+    } else if (n_cap < (3u << 20)) {
+        p->threads = 1024;
+        p->items = 4;
+        per = 2048;
+        most = kMaxBuckets;
+    } else {
+        p->threads = 1024;
+        p->items = 8;
+        per = 4096;
+        most = kMaxBuckets;
+    }
+    const uint64_t want = std::max<uint64_t>(1, n_cap / per);
+    used = std::max<uint64_t>(1, std::min<uint64_t>(used, bins));
+    while ((used >> (p->shift + 1)) >= want && (2u << p->shift) <= kMaxBins) ++p->shift;
+    auto buckets = [&] { return ((uint64_t)bins + (1ull << p->shift) - 1) >> p->shift; };
+    while (buckets() > most && (2u << p->shift) <= kMaxBins) ++p->shift;
+    const uint64_t nb = buckets();
+    if (nb > most) return false;
+    p->buckets = (uint32_t)nb;
+    p->tiles = ceil_div(n_cap, p->threads * p->items);
+    // the tables fit the scratch that every bin sort of this size has
+    if ((uint64_t)p->tiles * p->buckets > n_cap) return false;
+    if ((uint64_t)p->tiles + 2ull * p->buckets + 8ull > n_cap / 2) return false;
+    return true;
+}
+
+template <uint32_t BT, uint32_t ITEMS, uint32_t MAXB, uint32_t S>
+static int launch_passes(const BucketArgs& a, const VarTable& vt, hipStream_t st) {
+    constexpr uint32_t kWindow = BT * S / 2u;
+    hipLaunchKernelGGL((k_bucket_count<BT, ITEMS>), dim3(a.tiles), dim3(BT), 0, st, a);
+    FGX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_bucket_prefix, dim3(ceil_div(a.buckets, 64)), dim3(1024), 0, st, a);
+    FGX_HIP(hipGetLastError());
+    hipLaunchKernelGGL((k_bucket_split<BT, ITEMS, MAXB>), dim3(a.tiles), dim3(BT), 0, st, a, vt);
+    FGX_HIP(hipGetLastError());
+    // a bucket of m elements has (m - 1) / kWindow pieces after its first
+    hipLaunchKernelGGL((k_bucket_sort<BT, kMaxBins, S>), dim3(a.buckets + a.n_cap / kWindow), dim3(BT), 0, st, a, vt);
+    FGX_HIP(hipGetLastError());
+    return FGX_OK;
+}
+
+int bucket_sort(const BucketPlan& p, const KeyArgs& ka, uint32_t bins, const uint32_t* d_n, uint32_t n_cap, const float* x,
+                const float* y, const float* z, const VarTable& vt, uint32_t* start_out, uint32_t* words_a,
+                uint32_t* words_b, uint32_t* words_c, hipStream_t st) {
+    BucketArgs a{};
+    a.ka = ka;
+    a.d_n = d_n;
+    a.n_cap = n_cap;
+    a.shift = p.shift;
+    a.buckets = p.buckets;
+    a.tiles = p.tiles;
+    a.bins = bins;
+    a.x = x;
+    a.y = y;
+    a.z = z;
+    a.start_out = start_out;
+    if (p.one_block) {
+        hipLaunchKernelGGL((k_sort_one_block<1024, kMaxBins, kOneBlockMax / 1024u>), dim3(1), dim3(1024), 0, st, a, vt);
+        FGX_HIP(hipGetLastError());
+        return FGX_OK;
+    }
+    // words_a: n_cap 16-bit bins, then the small tables; words_b: indices; words_c: the counts
+    a.fine = reinterpret_cast<uint16_t*>(words_a);
+    uint32_t* tables = words_a + (n_cap + 1u) / 2u;
+    a.stage = tables;
+    a.totals = tables + 4;
+    a.starts = a.totals + p.buckets;
+    a.met = a.starts + p.buckets + 1;
+    a.idx = words_b;
+    a.counts = words_c;
+    // Elements of a tile that share a bucket lie next to each other in it; below 16 of them
+    // (a half cache line of a 4-byte variable) gathering from the whole list costs more than
+    // moving the variables twice, once the list is larger than the L2s hold.
+    if (p.items == 8 && p.shift) a.stage_above = ceil_div(n_cap, 16u);
+    if (p.threads == 256) return launch_passes<256, 4, 1024, 8>(a, vt, st);
+    if (p.items == 4) return launch_passes<1024, 4, kMaxBuckets, 8>(a, vt, st);
+    return launch_passes<1024, 8, kMaxBuckets, 16>(a, vt, st);
+}
+
+}  // namespace fgx

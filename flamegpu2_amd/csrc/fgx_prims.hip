@@ -11,7 +11,9 @@
 //   reduction          : fixed-shape (deterministic) tree
 //
 // Nothing here allocates or synchronises with the host.
+#include "fgx_bucket_sort.h"
 #include "fgx_internal.h"
+#include "fgx_keys.h"
 
 #include <algorithm>
 #include <cstring>
@@ -21,60 +23,6 @@ namespace fgx {
 constexpr uint32_t kBlock = 256;
 constexpr uint32_t kItems = 8;
 constexpr uint32_t kTile = kBlock * kItems;   // 2048 items per scan / compaction tile
-
-__device__ __forceinline__ uint32_t load_count(const uint32_t* d_n, uint32_t n_cap) {
-    if (!d_n) return n_cap;
-    const uint32_t n = __hip_atomic_load(d_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return n < n_cap ? n : n_cap;
-}
-
-// ================================================================ bin keys
-struct KeyArgs {
-    int32_t mode;        // 0: message bin (clamped, MessageSpatial3DDevice.cuh:646-672)
-                         // 1: agent sort key (unclamped, CUDASimulation.cu:372-408)
-                         // 2: bucket key, x holds int32 keys (MessageBucket.cu:58-72)
-    int32_t dims;
-    float min[3];
-    float radius;
-    float width[3];
-    uint32_t grid[3];
-    uint32_t key_mask;   // mode 1: (1 << key_bits) - 1
-    int32_t key_min;     // mode 2: lowest key
-    uint32_t keys;       // mode 2: number of keys
-};
-
-__device__ __forceinline__ uint32_t bin_key(const KeyArgs& k, float x, float y, float z) {
-    if (k.mode == 2) {
-        // keys outside the range were reported by setKey; clamp so they stay in the table
-        const int v = __float_as_int(x) - k.key_min;
-        return v < 0 ? 0u : ((uint32_t)v >= k.keys ? k.keys - 1u : (uint32_t)v);
-    }
-    if (k.mode == 0) {
-        int c[3];
-        const float p[3] = {x, y, z};
-        for (int a = 0; a < 3; ++a) {
-            if (a < k.dims) {
-                const int g = (int)floorf((p[a] - k.min[a]) / k.radius);
-                const int hi = (int)k.grid[a] - 1;
-                c[a] = g < 0 ? 0 : (g > hi ? hi : g);
-            } else {
-                c[a] = 0;
-            }
-        }
-        return (uint32_t)c[2] * k.grid[0] * k.grid[1] + (uint32_t)c[1] * k.grid[0] + (uint32_t)c[0];
-    } else {
-        const int gx = (int)floorf(((x - k.min[0]) / k.width[0]) * (float)k.grid[0]);
-        const int gy = (int)floorf(((y - k.min[1]) / k.width[1]) * (float)k.grid[1]);
-        uint32_t b;
-        if (k.dims == 3) {
-            const int gz = (int)floorf(((z - k.min[2]) / k.width[2]) * (float)k.grid[2]);
-            b = (uint32_t)gz * k.grid[0] * k.grid[1] + (uint32_t)gy * k.grid[0] + (uint32_t)gx;
-        } else {
-            b = (uint32_t)gy * k.grid[0] + (uint32_t)gx;
-        }
-        return b & k.key_mask;
-    }
-}
 
 // Histogram with wave-level run aggregation: consecutive lanes with equal keys
 // (the common case, as agents are kept in bin order) issue one atomic per run.
@@ -1171,12 +1119,17 @@ static int run_scan(const uint32_t* in, uint32_t* out, uint32_t n, char* scratch
     return scan_counts(in, out, n, hdr, status, (hipStream_t)stream);
 }
 
-// Shared by the message build and the agent sort.  shared_space: the working space is the
-// library's own per-GPU array (fgx_spatial_build_noalloc), which every such call shares:
-// its histogram is always cleared and no clean record is kept for it.
-static int run_bin_sort(fgx_ctx* ctx, const KeyArgs& ka, uint32_t bins, const uint32_t* d_n, uint32_t n_cap,
+// Shared by the message build, the bucket index and the agent sort.  used: about how many of
+// the bins occur; starts_read: whether anybody reads start_out.  shared_space: the working
+// space is the library's own per-GPU array (fgx_spatial_build_noalloc), which every such call
+// shares: its histogram is always cleared and no clean record is kept for it.
+//
+// Lists whose sizes bucket_plan() takes are sorted through LDS (fgx_bucket_sort.hip); sparse
+// tables (more bins than 1,024 per bucket allows for the list) and lists beyond 12 M elements
+// go through global atomics below.
+static int run_bin_sort(fgx_ctx* ctx, const KeyArgs& ka, uint32_t bins, uint64_t used, const uint32_t* d_n, uint32_t n_cap,
                         const float* x, const float* y, const float* z, const VarTable& vt, uint32_t* start_out,
-                        void* scratch, size_t scratch_bytes, void* stream, bool shared_space = false) {
+                        bool starts_read, void* scratch, size_t scratch_bytes, void* stream, bool shared_space = false) {
     const BuildLayout L = build_layout(n_cap, bins);
     if (!scratch || scratch_bytes < L.total) return fail(FGX_ERR_CAPACITY, "scratch too small for bin sort");
     char* s = static_cast<char*>(scratch);
@@ -1200,18 +1153,26 @@ static int run_bin_sort(fgx_ctx* ctx, const KeyArgs& ka, uint32_t bins, const ui
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     FGX_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
     const bool capturing = cap != hipStreamCaptureStatusNone;
+    //
+    // The bucket sort works in the key arrays only and leaves the histogram region of its own
+    // bin count as it found it.
     bool clean = false;
     const bool record = ctx && ctx->c.keep_zero && !shared_space;
+    BucketPlan plan;
+    const bool buckets = bucket_plan(n_cap, bins, used, &plan);
     if (record) {
         std::lock_guard<std::mutex> lk(clean_mutex());
         auto it = clean_record().find(scratch);
+        const bool zero = it != clean_record().end() && (it->second == bins || it->second == kAllZero);
         auto hit = bins_history().find(scratch);
         const bool single = hit != bins_history().end() && hit->second == bins;
-        clean = capturing ? single : (it != clean_record().end() && (it->second == bins || it->second == kAllZero));
+        clean = capturing ? single : zero;
         if (it != clean_record().end()) clean_record().erase(it);   // re-recorded once every launch is enqueued
+        if (buckets && zero && !capturing) clean_record()[scratch] = bins;
         if (hit == bins_history().end()) bins_history()[scratch] = bins;
         else if (hit->second != bins) hit->second = kMixedBins;
     }
+    if (buckets) return bucket_sort(plan, ka, bins, d_n, n_cap, x, y, z, vt, starts_read ? start_out : nullptr, key, sub, tmp, st);
     int rc = FGX_OK;
     if (!clean) {
         rc = fgx_fill_u32(hist, 0u, (size_t)bins + 2, stream);
@@ -1397,7 +1358,7 @@ static int spatial_build(fgx_ctx* ctx, const fgx_spatial_meta* meta, const uint3
         ka.width[a] = meta->width[a];
         ka.grid[a] = meta->grid[a] ? meta->grid[a] : 1u;
     }
-    return run_bin_sort(ctx, ka, meta->bins, d_n, n_cap, x, y, z, vt, pbm, scratch, scratch_bytes, stream);
+    return run_bin_sort(ctx, ka, meta->bins, meta->bins, d_n, n_cap, x, y, z, vt, pbm, true, scratch, scratch_bytes, stream);
 }
 
 int fgx_spatial_build(fgx_ctx* ctx, const fgx_spatial_meta* meta, const uint32_t* d_n, uint32_t n_cap,
@@ -1451,8 +1412,8 @@ int fgx_spatial_build_noalloc(fgx_ctx* ctx, const fgx_spatial_meta* meta, const 
         ka.width[a] = meta->width[a];
         ka.grid[a] = meta->grid[a] ? meta->grid[a] : 1u;
     }
-    return run_bin_sort(ctx, ka, meta->bins, d_n, n_cap, x, y, z, vt, pbm, space, FGX_NOALLOC_BUILD_BYTES, stream,
-                        true);
+    return run_bin_sort(ctx, ka, meta->bins, meta->bins, d_n, n_cap, x, y, z, vt, pbm, true, space, FGX_NOALLOC_BUILD_BYTES,
+                        stream, true);
 }
 
 int fgx_bucket_build(fgx_ctx* ctx, int32_t key_min, uint32_t keys, const uint32_t* d_n, uint32_t n_cap, const int32_t* key,
@@ -1470,7 +1431,7 @@ int fgx_bucket_build(fgx_ctx* ctx, int32_t key_min, uint32_t keys, const uint32_
     ka.key_min = key_min;
     ka.keys = keys;
     const float* kf = reinterpret_cast<const float*>(key);
-    return run_bin_sort(ctx, ka, keys, d_n, n_cap, kf, kf, nullptr, vt, pbm, scratch, scratch_bytes, stream);
+    return run_bin_sort(ctx, ka, keys, keys, d_n, n_cap, kf, kf, nullptr, vt, pbm, true, scratch, scratch_bytes, stream);
 }
 
 int fgx_array_build(fgx_ctx* ctx, uint32_t length, const uint32_t* d_n, uint32_t n_cap, const uint32_t* index,
@@ -1528,7 +1489,8 @@ int fgx_agent_sort(fgx_ctx* ctx, int dims, const float* mn, const float* mx, flo
     if (!scratch || scratch_bytes < L.total + align256((size_t)(bins + 1) * 4))
         return fail(FGX_ERR_CAPACITY, "fgx_agent_sort: scratch too small");
     auto* start = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) + L.total);
-    return run_bin_sort(ctx, ka, bins, d_n, n_cap, x, y, z, vt, start, scratch, L.total, stream);
+    return run_bin_sort(ctx, ka, bins, (uint64_t)ka.grid[0] * ka.grid[1] * ka.grid[2], d_n, n_cap, x, y, z, vt, start, false,
+                        scratch, L.total, stream);
 }
 
 int fgx_pack_records(const uint32_t* d_n, uint32_t n_cap, const void* w0, const void* w1, const void* w2,

@@ -639,6 +639,94 @@ def test_reduce_stats(ctx, code, dtype, acc, n):
     assert abs(sq - ref) <= 1e-10 * max(ref, 1.0)
 
 
+def _index_case(ctx, what, dims, n, bins_axis, positions, by, use_dn=None):
+    """Message index, agent sort or bucket index of one list against the oracle's keys and a
+    stable argsort: every variable, the records and the bin starts."""
+    from flamegpu2_amd import fgx
+    rng = np.random.default_rng(n + 7 * dims)
+    r = np.float32(0.5)
+    w = float(r) * bins_axis
+    m = n if use_dn is None else use_dn
+    if what == "bucket":
+        keys_all = (positions(rng, n)[0] * bins_axis).astype(np.int32).clip(-2, bins_axis + 1)
+        P, keys, bins = [keys_all.view(np.float32)], keys_all[:m].clip(0, bins_axis - 1), bins_axis
+    else:
+        P = [(p * w).astype(np.float32) for p in positions(rng, n)[:dims]]
+        if what == "agents":
+            keys, bits = O.agent_sort_keys(dims, [0.0] * dims, [w] * dims, float(r), P[0][:m], P[1][:m],
+                                           P[2][:m] if dims == 3 else None)
+            bins = 1 << bits
+        else:
+            meta = fgx.spatial_meta(dims, [0.0] * dims, [w] * dims, float(r))
+            bins = meta.bins
+            c = [np.clip(np.floor(p[:m] / r).astype(np.int64), 0, meta.grid[a] - 1) for a, p in enumerate(P)]
+            keys = c[0] + meta.grid[0] * (c[1] + (meta.grid[1] * c[2] if dims == 3 else 0))
+    order = np.argsort(np.asarray(keys).astype(np.int64), kind="stable")
+    raw = [p.view(np.uint8).reshape(n, 4) for p in P] + [rng.integers(0, 256, size=(n, b), dtype=np.uint8) for b in by]
+    sizes = [a.shape[1] for a in raw]
+    d_in = [dev(a.reshape(-1)) for a in raw]
+    d_out = [empty(n * b, np.uint8) for b in sizes]
+    d_n = dev(np.array([m], np.uint32)) if use_dn is not None else None
+    dn = ptr(d_n) if use_dn is not None else None
+    vi, vo = [ptr(t) for t in d_in], [ptr(t) for t in d_out]
+    op = fgx.FGX_OP_AGENT_SORT if what == "agents" else fgx.FGX_OP_SPATIAL_BUILD
+    sb = fgx.scratch_bytes(op, n, bins)
+    s = scratch(sb)
+    pbm, rec = empty(bins + 1, np.uint32), empty(4 * n, np.uint32)
+    xyz = vi[:dims] + [None] * (3 - dims)
+    if what == "agents":
+        fgx.agent_sort(ctx, dims, [0.0] * dims, [w] * dims, float(r), n, *xyz, vi, vo, sizes, ptr(s), sb, d_n=dn)
+    elif what == "bucket":
+        fgx.bucket_build(ctx, 0, bins, n, vi[0], vi, vo, sizes, ptr(pbm), ptr(s), sb, d_n=dn)
+    else:
+        fgx.spatial_build_records(ctx, meta, n, *xyz, vi, vo, sizes, [0, 1, 2 if dims == 3 else -1, dims], ptr(rec),
+                                  ptr(pbm), ptr(s), sb, d_n=dn)
+    sync()
+    for v, b in enumerate(sizes):
+        got = host(d_out[v], np.uint8, n * b).reshape(n, b)
+        assert np.array_equal(got[:m], raw[v][:m][order]), f"variable {v} ({b} bytes)"
+        assert not got[m:].any()
+    if what != "agents":
+        exp = np.concatenate([[0], np.cumsum(np.bincount(keys, minlength=bins))])
+        assert np.array_equal(host(pbm, np.uint32, bins + 1), exp)
+    if what == "messages":
+        got = host(rec, np.uint8, 16 * n).reshape(n, 4, 4)
+        for k, v in enumerate([0, 1, 2 if dims == 3 else -1, dims]):
+            exp = raw[v][:m][order] if v >= 0 else np.zeros((m, 4), np.uint8)
+            assert np.array_equal(got[:m, k], exp), f"record word {k}"
+
+
+def _uniform(rng, n):
+    return [rng.uniform(0, 1, n) for _ in range(3)]
+
+
+def _clumped(rng, n):
+    # most of the list in a thousandth of the space, some of it in one point
+    p = [np.where(np.arange(n) % 8 == 0, rng.uniform(0, 1, n), 0.4 + 0.1 * rng.uniform(0, 1, n)) for _ in range(3)]
+    for a in p:
+        a[n // 3:n // 2] = 0.77
+    return p
+
+
+@pytest.mark.parametrize("what,dims,n,axis,positions,use_dn", [
+    # one block: the smallest lists, its largest, one bin and the most bins
+    ("messages", 3, 1, 3, _uniform, None), ("messages", 2, 65, 1, _uniform, None), ("agents", 3, 4095, 9, _uniform, None),
+    ("messages", 3, 4096, 10, _clumped, None), ("bucket", 1, 4096, 1024, _uniform, 0), ("messages", 2, 4000, 32, _uniform, 1777),
+    # blocks of 256 threads: a tile and a wave more, odd sizes, few bins and a sparse table
+    ("messages", 3, 4097, 10, _uniform, None), ("agents", 2, 16384 + 63, 40, _uniform, None), ("bucket", 1, 30001, 7, _uniform, None),
+    ("messages", 3, 100003, 30, _uniform, 65537), ("messages", 3, 200000, 60, _clumped, None), ("bucket", 1, 262143, 300, _clumped, None),
+    ("messages", 3, 20000, 10, _uniform, 0),
+    # blocks of 1,024 threads, and buckets shared by several blocks
+    ("messages", 3, 262144, 20, _uniform, None), ("agents", 3, 524289, 41, _uniform, 300001), ("messages", 2, 1000003, 200, _clumped, None),
+    ("agents", 3, 700001, 64, _clumped, None), ("bucket", 1, 400000, 3, _uniform, None),
+    # lists in no order and in order from 3 M elements on; whole and clumped
+    ("messages", 2, 3145728 + 5, 400, _uniform, None), ("agents", 2, 3500000, 410, _uniform, 3300001),
+    ("messages", 2, 3200001, 400, _clumped, None), ("bucket", 1, 3145728, 50000, lambda rng, n: [np.sort(rng.uniform(0, 1, n))], None)])
+def test_index_sizes_and_shapes(ctx, what, dims, n, axis, positions, use_dn):
+    by = [4, 4, 8, 4, 2, 4, 4, 4, 12] if n < 300000 else [4, 8, 1]
+    _index_case(ctx, what, dims, n, axis, positions, by, use_dn)
+
+
 @pytest.mark.parametrize("n", [1, 1023, 1025, 200 * 1024, 200 * 1024 + 1, 8 * 200 * 1024 - 1, 8 * 200 * 1024 + 3])
 def test_reduce_stats_block_edges(ctx, n):
     # sizes around the blocks and batches of the one-pass statistics, on values far from zero
