@@ -88,6 +88,8 @@ class BatchSimulation {
     std::vector<int> finished() const;
     unsigned int stepsDone(int h) const { return sim(h).steps_done; }
     void getPopulationData(int h, AgentVector& pop);
+    // The population straight into host arrays (name, array of count x bytes); returns the count.
+    uint32_t readPopulation(int h, const std::string& agent, const std::vector<std::pair<std::string, void*>>& dst);
     void remove(int h);
     void setTuning(const Tuning& t);
     const Tuning& tuning() const { return tuning_; }
@@ -252,6 +254,7 @@ class BatchSimulation {
     std::vector<void*> buffer_state() const;
     void set_buffer_state(const std::vector<void*>& st);
     void check_errors(const Sim& s, uint32_t slot);
+    const List& part(const Sim& s, const std::string& agent, uint32_t* off, uint32_t* n);
 
     std::shared_ptr<ModelData> m_;
     int device_ = 0;
@@ -1548,6 +1551,25 @@ inline void BatchSimulation::check_errors(const Sim& s, uint32_t slot) {
                                                     e[0], detail::device_error_text(e[0]), s.handle, e[1], e[2]));
 }
 
+// Place and size of a resident simulation's part of an agent list, after the work enqueued so far.
+inline const BatchSimulation::List& BatchSimulation::part(const Sim& s, const std::string& agent, uint32_t* off, uint32_t* n) {
+    synchronize();
+    uint32_t slot = 0;
+    while (slot < order_.size() && order_[slot] != s.handle) ++slot;
+    check_errors(s, slot);
+    auto it = agents_.find(agent);
+    if (it == agents_.end()) throw exception::InvalidAgentName("BatchSimulation: unknown agent");
+    const List& l = it->second.list;
+    *n = l.cnt[slot];
+    *off = l.off[slot];
+    if (dynamic_) {
+        detail::fgx_check(fgx_memcpy_d2h(n, l.d_cnt + slot, 4, stream_), "count readback");
+        detail::fgx_check(fgx_memcpy_d2h(off, l.d_off + slot, 4, stream_), "offset readback");
+        synchronize();
+    }
+    return l;
+}
+
 inline void BatchSimulation::getPopulationData(int h, AgentVector& pop) {
     Sim& s = sim(h);
     if (!s.resident) {
@@ -1556,19 +1578,8 @@ inline void BatchSimulation::getPopulationData(int h, AgentVector& pop) {
         pop = *it->second;
         return;
     }
-    synchronize();
-    uint32_t slot = 0;
-    while (slot < order_.size() && order_[slot] != h) ++slot;
-    check_errors(s, slot);
-    auto it = agents_.find(pop.getAgentName());
-    if (it == agents_.end()) throw exception::InvalidAgentName("BatchSimulation: unknown agent");
-    const List& l = it->second.list;
-    uint32_t n = l.cnt[slot], o = l.off[slot];
-    if (dynamic_) {
-        detail::fgx_check(fgx_memcpy_d2h(&n, l.d_cnt + slot, 4, stream_), "count readback");
-        detail::fgx_check(fgx_memcpy_d2h(&o, l.d_off + slot, 4, stream_), "offset readback");
-        synchronize();
-    }
+    uint32_t n = 0, o = 0;
+    const List& l = part(s, pop.getAgentName(), &o, &n);
     pop.resize(n);
     for (auto& v : l.vars)
         if (n)
@@ -1578,6 +1589,28 @@ inline void BatchSimulation::getPopulationData(int h, AgentVector& pop) {
     synchronize();
 }
 
+inline uint32_t BatchSimulation::readPopulation(int h, const std::string& agent,
+                                                const std::vector<std::pair<std::string, void*>>& dst) {
+    Sim& s = sim(h);
+    if (!s.resident) {
+        auto it = s.pop.find(agent);
+        if (it == s.pop.end()) throw exception::InvalidAgentName("BatchSimulation: unknown agent");
+        for (auto& d : dst) std::memcpy(d.second, it->second->raw(d.first).data(), it->second->raw(d.first).size());
+        return (uint32_t)it->second->size();
+    }
+    uint32_t n = 0, o = 0;
+    const List& l = part(s, agent, &o, &n);
+    for (auto& d : dst) {
+        const detail::VarBuf* b = nullptr;
+        for (auto& v : l.vars)
+            if (v.name == d.first) b = &v;
+        if (!b) throw exception::InvalidAgentVar("BatchSimulation: agent '" + agent + "' has no variable '" + d.first + "'");
+        detail::fgx_check(fgx_memcpy_d2h(d.second, (const char*)b->cur + (size_t)o * b->bytes, (size_t)n * b->bytes, stream_),
+                          "population download");
+    }
+    if (!dst.empty()) synchronize();
+    return n;
+}
 
 // include/flamegpu/simulation/CUDAEnsemble.h:40-129.  simulate() runs the plans in one
 // BatchSimulation when the model can be batched (the default; Config().batched = false

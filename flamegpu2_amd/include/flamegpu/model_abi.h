@@ -65,6 +65,15 @@ inline std::shared_ptr<flamegpu::AgentData> agent(fgxm_sim* s, const char* name)
 }  // namespace fgxm_detail
 
 namespace fgxm_detail {
+// Where a population read goes: the caller's array of each declared variable it wants, and the IDs.
+inline std::vector<std::pair<std::string, void*>> targets(const flamegpu::AgentData& a, void* const* vars, uint32_t* ids) {
+    std::vector<std::pair<std::string, void*>> t;
+    for (size_t v = 0; v < a.declared.size(); ++v)
+        if (vars[v]) t.emplace_back(a.declared[v], vars[v]);
+    if (ids) t.emplace_back("_id", ids);
+    return t;
+}
+
 inline void var_info(const std::shared_ptr<flamegpu::AgentData>& a, uint32_t v, const char** name, int32_t* type,
                      uint32_t* elements, uint32_t* bytes) {
     {
@@ -156,13 +165,7 @@ FGXM_EXPORT int fgxm_count(fgxm_sim* s, const char* agent, const char* state, ui
 FGXM_EXPORT int fgxm_get_agents(fgxm_sim* s, const char* agent, const char* state, void* const* vars, uint32_t* ids) {
     return fgxm_detail::guard([&] {
         auto a = fgxm_detail::agent(s, agent);
-        flamegpu::AgentVector pop{flamegpu::AgentDescription(a)};
-        s->sim->getPopulationData(pop, state ? state : "");
-        for (size_t v = 0; v < a->declared.size(); ++v) {
-            auto& raw = pop.raw(a->declared[v]);
-            if (vars[v]) std::memcpy(vars[v], raw.data(), raw.size());
-        }
-        if (ids) std::memcpy(ids, pop.raw("_id").data(), pop.size() * 4);
+        s->sim->readPopulation(a->name, state ? state : "", fgxm_detail::targets(*a, vars, ids));
     });
 }
 
@@ -640,22 +643,14 @@ FGXM_EXPORT int fgxm_batch_steps_done(fgxm_batch* b, int32_t h, uint32_t* steps)
 FGXM_EXPORT int fgxm_batch_count(fgxm_batch* b, int32_t h, const char* agent, uint32_t* n) {
     return fgxm_detail::guard([&] {
         auto a = fgxm_detail::batch_agent(b, agent);
-        flamegpu::AgentVector pop{flamegpu::AgentDescription(a)};
-        b->batch->getPopulationData(fgxm_detail::handle(b, h), pop);
-        *n = (uint32_t)pop.size();
+        *n = b->batch->readPopulation(fgxm_detail::handle(b, h), a->name, {});
     });
 }
 
 FGXM_EXPORT int fgxm_batch_get_agents(fgxm_batch* b, int32_t h, const char* agent, void* const* vars, uint32_t* ids) {
     return fgxm_detail::guard([&] {
         auto a = fgxm_detail::batch_agent(b, agent);
-        flamegpu::AgentVector pop{flamegpu::AgentDescription(a)};
-        b->batch->getPopulationData(fgxm_detail::handle(b, h), pop);
-        for (size_t v = 0; v < a->declared.size(); ++v) {
-            auto& raw = pop.raw(a->declared[v]);
-            if (vars[v]) std::memcpy(vars[v], raw.data(), raw.size());
-        }
-        if (ids) std::memcpy(ids, pop.raw("_id").data(), pop.size() * 4);
+        b->batch->readPopulation(fgxm_detail::handle(b, h), a->name, fgxm_detail::targets(*a, vars, ids));
     });
 }
 

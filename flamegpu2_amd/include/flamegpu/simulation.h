@@ -606,6 +606,11 @@ class CUDASimulation {
     // src/flamegpu/simulation/CUDASimulation.cu:1418-1452
     void setPopulationData(AgentVector& pop, const std::string& state = "");
     void getPopulationData(AgentVector& pop, const std::string& state = "");
+    // The population of (agent, state) straight into host arrays: dst holds, for each variable
+    // wanted, its name and an array of count x bytes (getPopulationData without the AgentVector
+    // between).  Returns the count.
+    uint32_t readPopulation(const std::string& agent, const std::string& state,
+                            const std::vector<std::pair<std::string, void*>>& dst);
     void synchronize() {
         if (stream_) detail::fgx_check(fgx_stream_synchronize(stream_), "stream synchronize");
     }
@@ -1656,6 +1661,26 @@ inline void CUDASimulation::getPopulationData(AgentVector& pop, const std::strin
             detail::fgx_check(fgx_memcpy_d2h(pop.raw(v.name).data(), v.cur, (size_t)l.h_count * v.bytes, stream_),
                               "population download");
     synchronize();
+}
+
+inline uint32_t CUDASimulation::readPopulation(const std::string& agent, const std::string& state_in,
+                                               const std::vector<std::pair<std::string, void*>>& dst) {
+    ensure_init();
+    auto& a = agent_rt(agent);
+    const std::string state = state_in.empty() ? a.d->initial_state : state_in;
+    auto it = a.states.find(state);
+    if (it == a.states.end()) throw exception::InvalidAgentState("Agent '" + a.d->name + "' has no state '" + state + "'");
+    sync_counts();
+    auto& l = it->second;
+    check_device_error();
+    for (auto& d : dst) {
+        const int vi = l.var_index(d.first);
+        if (vi < 0) throw exception::InvalidAgentVar("Agent '" + a.d->name + "' does not contain variable '" + d.first + "'");
+        detail::fgx_check(fgx_memcpy_d2h(d.second, l.vars[vi].cur, (size_t)l.h_count * l.vars[vi].bytes, stream_),
+                          "population download");
+    }
+    synchronize();
+    return l.h_count;
 }
 
 inline void CUDASimulation::check_device_error() {

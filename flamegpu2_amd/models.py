@@ -148,8 +148,8 @@ class Simulation:
     def get_agents(self, agent, state=None):
         info = self.var_info(agent)
         n = self.count(agent, state)
-        outs = [np.zeros(n * e, dtype=dt) for (_, dt, e, _) in info]
-        ids = np.zeros(n, dtype=np.uint32)
+        outs = [np.empty(n * e, dtype=dt) for (_, dt, e, _) in info]   # written whole by the read
+        ids = np.empty(n, dtype=np.uint32)
         vp = (ctypes.c_void_p * max(len(outs), 1))(*[o.ctypes.data for o in outs])
         self._chk(self.L.fgxm_get_agents(self.h, _b(agent), _b(state), vp,
                                          ids.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))))
@@ -342,8 +342,8 @@ class Batch:
         info = self.var_info(agent)
         n = ctypes.c_uint32()
         self._chk(self.L.fgxm_batch_count(self.h, handle, _b(agent), ctypes.byref(n)))
-        outs = [np.zeros(n.value * e, dtype=dt) for (_, dt, e, _) in info]
-        ids = np.zeros(n.value, dtype=np.uint32)
+        outs = [np.empty(n.value * e, dtype=dt) for (_, dt, e, _) in info]   # written whole by the read
+        ids = np.empty(n.value, dtype=np.uint32)
         vp = (ctypes.c_void_p * max(len(outs), 1))(*[o.ctypes.data for o in outs])
         self._chk(self.L.fgxm_batch_get_agents(self.h, handle, _b(agent), vp,
                                                ids.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))))
