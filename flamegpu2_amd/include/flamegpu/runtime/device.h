@@ -1553,15 +1553,27 @@ __device__ __forceinline__ void run_agent(const ThreadCtx& c) {
 }
 
 // Workgroups go to the 8 XCDs round-robin (workgroup w runs on XCD w % 8), and each
-// XCD has its own L2.  This renumbering gives XCD x one contiguous range of logical
-// blocks, started in order, so the bin-sorted agents that share neighbourhoods (and
-// so messages) also share an L2: XCD x gets q + (x < r) blocks, q = G / 8, r = G % 8,
-// starting at x*q + min(x, r).
-__device__ __forceinline__ uint32_t xcd_block() {
-    constexpr uint32_t kXcds = 8;
-    const uint32_t g = gridDim.x, b = blockIdx.x;
-    const uint32_t x = b % kXcds, k = b / kXcds, q = g / kXcds, r = g % kXcds;
-    return x * q + (x < r ? x : r) + k;
+// XCD has its own L2.  This renumbering gives XCD x one contiguous range of the `blocks`
+// logical blocks, started in order, so the bin-sorted agents that share neighbourhoods (and
+// so messages) also share an L2: XCD x gets q + (x < r) blocks, q = blocks / 8,
+// r = blocks % 8, starting at x*q + min(x, r).  Workgroup `k` of XCD `x`; kNoBlock behind
+// the XCD's last block, where the launch has more workgroups.
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kNoBlock = 0xFFFFFFFFu;
+__device__ __forceinline__ uint32_t xcd_block(uint32_t x, uint32_t k, uint32_t blocks) {
+    const uint32_t q = blocks / kXcds, r = blocks % kXcds;
+    return k < q + (x < r ? 1u : 0u) ? x * q + (x < r ? x : r) + k : kNoBlock;
+}
+__device__ __forceinline__ uint32_t xcd_block(uint32_t blocks) {
+    return xcd_block(blockIdx.x % kXcds, blockIdx.x / kXcds, blocks);
+}
+// The blocks that `n` agents fill.  Launches are sized for a list's capacity; the renumbering
+// runs over the blocks with agents: a list filled to 40 % would keep only 4 of the 8 XCDs busy
+// (predator-prey, 1 M prey and 250 k predators, lists about 40 % full: the layers' launches
+// 183 us on average that way, 110 so).  At least 1: block 0 writes the message count of an empty list.
+__device__ __forceinline__ uint32_t filled_blocks(uint32_t n) {
+    const uint32_t b = (__builtin_amdgcn_readfirstlane(n) + blockDim.x - 1u) / blockDim.x;
+    return b ? b : 1u;
 }
 
 // Agents [first, n) of the list run, first = the agents a function condition disabled.
@@ -1587,14 +1599,16 @@ __device__ __forceinline__ __attribute__((address_space(3))) uint32_t* wave_tabl
     return nullptr;
 }
 
-// One block of an agent-function launch: block `blk` of the function runs agents
-// [first + blk * blockDim, ...) of its list.  Shared by the function's own kernel (its
-// launch record in the kernel-argument segment) and the layer kernel (its record in
+// One workgroup of an agent-function launch, the k-th of XCD x's: block b of the function
+// runs agents [first + b * blockDim, ...) of its list.  Shared by the function's own kernel
+// (its launch record in the kernel-argument segment) and the layer kernel (its record in
 // device memory).
 template <typename F>
-__device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t blk) {
+__device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t x, uint32_t k) {
     const uint32_t first = a.d_first ? load_count(a.d_first) : 0u;
     const uint32_t n = a.d_n ? load_count(a.d_n) : a.n_cap;
+    const uint32_t blk = xcd_block(x, k, filled_blocks(n > first ? n - first : 0u));
+    if (blk == kNoBlock) return;
     const uint32_t o = blk * blockDim.x + threadIdx.x;
     if (a.d_msg_count_out && o == 0) *a.d_msg_count_out = n;   // one message per agent (no condition here)
     if (first + o >= n) return;
@@ -1608,14 +1622,14 @@ __device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t blk
 
 template <typename F>
 __global__ void __launch_bounds__(256) agent_function_kernel(const FnArgs a) {
-    run_function_block<F>(a, xcd_block());
+    run_function_block<F>(a, blockIdx.x % kXcds, blockIdx.x / kXcds);
 }
 
 // The same kernel built for 8 resident waves per SIMD (at most 64 VGPRs), for neighbour
 // walks: their loops wait on gathers, and a kernel a few registers above 64 keeps only 7.
 template <typename F>
 __global__ void __launch_bounds__(256, 8) agent_function_kernel_w8(const FnArgs a) {
-    run_function_block<F>(a, xcd_block());
+    run_function_block<F>(a, blockIdx.x % kXcds, blockIdx.x / kXcds);
 }
 
 // Whether a function's launches take agent_function_kernel_w8: when the plain build needs
@@ -1689,19 +1703,18 @@ struct fn_collect<Lo, Hi, true> {
 };
 
 template <typename... Fs, size_t... I>
-__device__ __forceinline__ void run_layer_fn(uint32_t fn, const FnArgs& a, uint32_t blk, std::index_sequence<I...>) {
-    ((fn == I ? run_function_block<Fs>(a, blk) : (void)0), ...);
+__device__ __forceinline__ void run_layer_fn(uint32_t fn, const FnArgs& a, uint32_t x, uint32_t k, std::index_sequence<I...>) {
+    ((fn == I ? run_function_block<Fs>(a, x, k) : (void)0), ...);
 }
 
-// One launch for the functions of a layer (fgx_layer_launch builds the image; function k
-// has begin[k + 1] - begin[k] blocks).  Each function's blocks are split evenly over the 8
-// XCDs, in contiguous chunks as xcd_block() gives a launch of its own (neighbouring agents
-// share an L2): workgroup w runs on XCD x = w % 8 as that XCD's block j = w / 8, and XCD x
-// runs function 0's chunk, then function 1's, and so on.  A whole-grid contiguous split
-// would put a small function's (mostly idle) blocks on some XCDs and the busy ones on others.
+// One launch for the functions of a layer (fgx_layer_launch builds the image; function f
+// has begin[f + 1] - begin[f] blocks).  Each function's blocks are split evenly over the 8
+// XCDs, in contiguous chunks as a launch of its own has them (neighbouring agents share an
+// L2): workgroup w runs on XCD x = w % 8 as that XCD's workgroup j = w / 8, and XCD x runs
+// function 0's share, then function 1's, and so on.  A whole-grid contiguous split would put
+// a small function's (mostly idle) blocks on some XCDs and the busy ones on others.
 template <typename... Fs>
 __global__ void __launch_bounds__(256) layer_kernel(const char* __restrict__ image) {
-    constexpr uint32_t kXcds = 8;
     const fgx_layer_header& h = *reinterpret_cast<const fgx_layer_header*>(image);
     const uint32_t x = blockIdx.x % kXcds;
     uint32_t j = blockIdx.x / kXcds;
@@ -1711,17 +1724,17 @@ __global__ void __launch_bounds__(256) layer_kernel(const char* __restrict__ ima
     for (uint32_t f = 0; f < FGX_LAYER_MAX_FNS; ++f) {
         if (f >= nf || k != FGX_LAYER_MAX_FNS) continue;
         const uint32_t nb = h.begin[f + 1] - h.begin[f];
-        const uint32_t lo = (uint32_t)(((uint64_t)x * nb) / kXcds), hi = (uint32_t)(((uint64_t)(x + 1) * nb) / kXcds);
-        if (j < hi - lo) {
+        const uint32_t share = nb / kXcds + (x < nb % kXcds ? 1u : 0u);
+        if (j < share) {
             k = f;
-            local = lo + j;
+            local = j;
         } else {
-            j -= hi - lo;
+            j -= share;
         }
     }
     if (k == FGX_LAYER_MAX_FNS) return;   // this XCD's share is done
     const FnArgs& a = *reinterpret_cast<const FnArgs*>(image + FGX_LAYER_ARGS_OFFSET + (size_t)k * h.stride);
-    run_layer_fn<Fs...>(h.fn[k], a, local, std::index_sequence_for<Fs...>{});
+    run_layer_fn<Fs...>(h.fn[k], a, x, local, std::index_sequence_for<Fs...>{});
 }
 
 // Batched launch: the simulations of a batch share one launch.  Tile t (blockDim x
@@ -1736,7 +1749,7 @@ __global__ void __launch_bounds__(1024) agent_function_kernel_seg(const FnArgs a
     // segs[nsegs] is the sentinel record: its tile_off is the batch's tile count, kept on
     // the device when births and deaths change the populations
     const uint32_t ntiles = segs[nsegs].tile_off;
-    const uint32_t lb = xcd_block();
+    const uint32_t lb = xcd_block(gridDim.x);
     const uint32_t t0 = (uint32_t)((uint64_t)lb * ntiles / gridDim.x);
     const uint32_t t1 = (uint32_t)((uint64_t)(lb + 1) * ntiles / gridDim.x);
     for (uint32_t t = t0; t < t1; ++t) {
@@ -1919,7 +1932,9 @@ __global__ void __launch_bounds__(256) agent_function_kernel_staged(const FnArgs
     extern __shared__ uint32_t fgx_stage_smem[];
     __shared__ StageHeader sh;
     const uint32_t n = a.d_n ? load_count(a.d_n) : a.n_cap;
-    const uint32_t b0 = xcd_block() * blockDim.x;
+    const uint32_t blk = xcd_block(filled_blocks(n));
+    if (blk == kNoBlock) return;
+    const uint32_t b0 = blk * blockDim.x;
     if (a.d_msg_count_out && b0 == 0 && threadIdx.x == 0) *a.d_msg_count_out = n;
     if (b0 >= n) return;
     const uint32_t i = b0 + threadIdx.x;

@@ -83,6 +83,26 @@ def test_boids_bit_exact(n, steps, graphs, staging, tables):
     _compare(sim, ref, 0, "Boid", exact=True)
 
 
+# Lists filled in part (blocks with agents spread over the XCDs), positions on the edges of
+# cells: exact against the oracle.
+@pytest.mark.parametrize("n,capacity", [(1, 1), (255, 9000), (2047, 2047), (2049, 2049), (2305, 40000), (70001, 300000),
+                                        (262161, 262161), (300000, 524800)])
+def test_boids_filled_blocks(n, capacity):
+    params, arrs = workloads.boids(capacity, seed=11)
+    sim = Simulation("boids_spatial3D", params, seed=11)
+    sim.set_agents("Boid", arrs)
+    arrs = [np.array(a[:n]) for a in arrs]
+    for k in range(3):
+        edge = np.round(arrs[k][k::5] / params[2]) * params[2]
+        arrs[k][k::5] = np.clip(edge, params[0], params[1])
+    sim.set_agents("Boid", arrs, ids=np.arange(1, n + 1))
+    ref = O.Sim(1, params, 11)
+    ref.set_agents(0, arrs)
+    sim.step(1)
+    ref.step(1)
+    _compare(sim, ref, 0, "Boid", exact=True)
+
+
 # fusion: the two functions of each layer as one launch (default) or one launch each
 @pytest.mark.parametrize("staging,tables,fusion", [(0, 1, 1), (1, 1, 1), (0, 0, 1), (0, 1, 0)])
 def test_predprey_small_bit_exact_traces(staging, tables, fusion):
