@@ -107,6 +107,11 @@ class BatchSimulation {
         unit_tables_ = on;
         clear_graphs();
     }
+    // 64-bit message addresses for lists of any size (CUDASimulation::setWideAddresses).
+    void setWideAddresses(bool on) {
+        wide_ = on;
+        clear_graphs();
+    }
     void setGraphs(bool on) {
         graphs_on_ = on;
         clear_graphs();
@@ -296,6 +301,7 @@ class BatchSimulation {
     float bin_mult_ = 1.0f;
     bool graphs_on_ = true;
     bool unit_tables_ = true;
+    bool wide_ = false;
     uint32_t stable_steps_ = 0;   // steps since the last repack
     bool dynamic_ = false;        // some function removes or adds agents
     uint32_t* d_word_ = nullptr;  // a count nobody reads (the births compaction's total)
@@ -1038,6 +1044,7 @@ inline void BatchSimulation::launch(FnB& f) {
     fill_table(a.agent, &a.agent_mul, l.vars, false);
     if (f.in) {
         fill_table(a.msg_in, &a.msg_in_mul, f.in->list.vars, false);
+        a.wide = wide_ || f.in->list.cap >= detail::kWideMessages ? 1 : 0;
         a.in_meta.packed = f.in->packed;   // covers the whole batch, indexed like the message arrays
     }
     if (f.out) {

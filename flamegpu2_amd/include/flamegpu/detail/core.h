@@ -230,6 +230,12 @@ inline const char* device_error_text(uint32_t code) {
     }
 }
 
+// Below this many messages every byte offset into a spatial list's arrays (elements of up to
+// 16 bytes) fits 32 bits: loads take a scalar base and a 32-bit lane offset, where 64-bit
+// addresses cost up to three vector instructions each.  Larger lists run kernels of their own
+// (agent_function_kernel_wide).
+constexpr uint32_t kWideMessages = 1u << 28;
+
 struct FnArgs {
     uint32_t n_cap;              // launch bound (state list capacity)
     const char* zero_page;       // 64 zero bytes: reads through an unresolved binding land here
@@ -249,6 +255,7 @@ struct FnArgs {
     const uint32_t* ids;         // the agent list's "_id" array
     const uint32_t* d_first;     // function condition: agents [*d_first, n) run (NULL: all)
     int32_t msg_out_optional;
+    int32_t wide;                // spatial input: the list may hold kWideMessages or more
     int32_t unit_tables;         // spatial input: build the per-wave unit tables in LDS (0: bin table from HBM)
     uint32_t* d_msg_count_out;   // mandatory output: the launch writes the message count (agent count) here
     uint32_t agent_mul, msg_in_mul, msg_out_mul, new_mul, env_mul;

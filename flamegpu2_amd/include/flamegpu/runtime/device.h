@@ -54,6 +54,7 @@ struct ThreadCtx {
     uint32_t lidx;              // index among the agents this launch runs (output slots, flags)
     uint32_t stream_id;         // RNG stream of the call
     __attribute__((address_space(3))) uint32_t* wtab;   // this wave's LDS region for spatial unit tables (null: none)
+    bool wide = false;          // the spatial message list holds kWideMessages or more (a constant of the kernel)
 };
 
 // Per-wave LDS region of the spatial iterators (kWaveTabWords words):
@@ -83,18 +84,24 @@ struct Bound {
 template <typename T>
 __device__ __forceinline__ Bound resolve(const VarBinding (&tab)[VAR_SLOTS], uint32_t mul, uint32_t h, uint32_t len,
                                          const ThreadCtx& c, uint32_t err_unknown, uint32_t err_type, bool write) {
-    // one 16-byte load of the whole binding, then selects on the values (a select
-    // of addresses would chain two dependent scalar loads)
+    // one 16-byte load of the whole binding
     const uint4 raw = *reinterpret_cast<const uint4*>(&tab[table_slot(h, mul, VAR_SLOT_BITS)]);
     // name hash and element bytes (whose reserved upper half-word is zero) checked by
     // one 64-bit compare against a compile-time constant; one branch to the report
     const uint64_t got = ((uint64_t)raw.y << 32) | raw.x;
     const uint64_t want = ((uint64_t)((uint32_t)sizeof(T) * len) << 32) | h;
     const bool ok = got == want;
-    if (__builtin_expect(!ok, 0)) report_error(c.err.d_error, raw.x != h ? err_unknown : err_type, h, c.err.index);
-    const uint64_t bound = ((uint64_t)raw.w << 32) | raw.z;
-    const uint64_t fallback = write ? (uint64_t)c.sink_page : (uint64_t)c.zero_page;
-    return Bound{ok ? bound : fallback, ok ? 0xFFFFFFFFu : 0u};
+    Bound b{((uint64_t)raw.w << 32) | raw.z, 0xFFFFFFFFu};
+    if (__builtin_expect(!ok, 0)) {
+        report_error(c.err.d_error, raw.x != h ? err_unknown : err_type, h, c.err.index);
+        // the empty asm keeps the end of the report's per-lane branch apart from the join below,
+        // so that the address merges two scalars and stays one
+        const uint64_t page = write ? (uint64_t)c.sink_page : (uint64_t)c.zero_page;
+        uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)page), hi = __builtin_amdgcn_readfirstlane((uint32_t)(page >> 32));
+        asm volatile("" : "+s"(lo), "+s"(hi));
+        b = Bound{((uint64_t)hi << 32) | lo, 0u};
+    }
+    return b;
 }
 
 template <typename T, unsigned N>
@@ -103,6 +110,17 @@ __device__ __forceinline__ T load_var(const VarBinding (&tab)[VAR_SLOTS], uint32
     const uint32_t h = name_hash(name, N);
     const Bound b = resolve<T>(tab, mul, h, 1, c, err_unknown, err_type, false);
     return b.as<const T>()[idx & b.mask];
+}
+
+// load_var for an element of a spatial message list.
+template <typename T, unsigned N>
+__device__ __forceinline__ T load_msg_var(const char (&name)[N], uint32_t idx, const ThreadCtx& c) {
+    const uint32_t h = name_hash(name, N);
+    const Bound b = resolve<T>(c.a.msg_in, c.a.msg_in_mul, h, 1, c, DERR_UNKNOWN_MSG_VAR, DERR_MSG_VAR_TYPE, false);
+    if (c.wide || sizeof(T) > 16) return b.as<const T>()[idx & b.mask];
+    uint32_t off = (idx * (uint32_t)sizeof(T)) & b.mask;
+    asm("" : "+v"(off));
+    return *(gptr<const T>)(b.addr + (uint64_t)off);
 }
 
 template <typename T, unsigned N>
@@ -423,6 +441,11 @@ constexpr uint32_t kHashId = name_hash("id", 3);
 // On the wave's unit table a lane starts with a bit mask of its non-empty units and
 // takes the lowest remaining one whenever its current unit ends.
 //
+// Over large lists the walk is bound by vector issue (boids, 1 M: 211 M wave instructions,
+// 118 a candidate, 343 us): scalar bases with 32-bit lane offsets (load_msg_var, fetch),
+// virtual coordinates only where a search can wrap (near_origin) and a shorter unit step
+// (take_unit) leave 176 M (95 a candidate) and, with blocks of 1024, 290 us.
+//
 // Source: the message list in HBM (bin table pbm, packed records), or, in the staged
 // kernel when every lane of the wave is covered by the block's LDS copy, the LDS tables
 // (units then name virtual bin entries and the look-ahead walks LDS slots).
@@ -457,7 +480,11 @@ class SpatialFilter {
         const bool id_ok = id_known && bi.bytes == 4;
         id_err_ = id_ok ? 0u : (id_known ? (uint32_t)detail::DERR_MSG_VAR_TYPE : (uint32_t)detail::DERR_UNKNOWN_MSG_VAR);
         pbm_ = m.pbm;
-        rec_ = reinterpret_cast<const uint4*>(c.a.in_meta.packed);   // the launch's (a batch: all simulations')
+        rec_ = reinterpret_cast<const char*>(c.a.in_meta.packed);   // the launch's (a batch: all simulations')
+        if (WRAP) {
+            flat_ = __builtin_amdgcn_readfirstlane(
+                __all(flat(m, 0, cx) && flat(m, 1, cy) && (DIMS == 2 || flat(m, 2, cz))) ? 1 : 0);
+        }
         sv_ = nullptr;
         tab_ = nullptr;
         tm_ = 0u;
@@ -508,17 +535,16 @@ class SpatialFilter {
                     return v;
                 }
             }
-            return detail::load_var<T>(f_.c_.a.msg_in, f_.c_.a.msg_in_mul, name, g_, f_.c_, detail::DERR_UNKNOWN_MSG_VAR,
-                                       detail::DERR_MSG_VAR_TYPE);
+            return detail::load_msg_var<T>(name, g_, f_.c_);
         }
         template <typename T, size_type L, unsigned N>
         __device__ __forceinline__ T getVariable(const char (&name)[N], unsigned int e) const {
             return detail::load_elem<T>(f_.c_.a.msg_in, f_.c_.a.msg_in_mul, name, g_, L, e, f_.c_,
                                         detail::DERR_UNKNOWN_MSG_VAR, detail::DERR_MSG_VAR_TYPE);
         }
-        __device__ __forceinline__ float getVirtualX() const { return getVirtualX(f_.loc_[0]); }
-        __device__ __forceinline__ float getVirtualY() const { return getVirtualY(f_.loc_[1]); }
-        __device__ __forceinline__ float getVirtualZ() const { return getVirtualZ(f_.loc_[2]); }
+        __device__ __forceinline__ float getVirtualX() const { return near_origin(0, x_); }
+        __device__ __forceinline__ float getVirtualY() const { return near_origin(1, y_); }
+        __device__ __forceinline__ float getVirtualZ() const { return near_origin(2, z_); }
         __device__ __forceinline__ float getVirtualX(float x1) const { return detail::virtual_coord(x_, x1, f_.width_[0]); }
         __device__ __forceinline__ float getVirtualY(float y1) const { return detail::virtual_coord(y_, y1, f_.width_[1]); }
         __device__ __forceinline__ float getVirtualZ(float z1) const { return detail::virtual_coord(z_, z1, f_.width_[2]); }
@@ -526,6 +552,15 @@ class SpatialFilter {
 
      private:
         friend class iterator;
+        // virtual_coord towards the search origin.  On an axis along which the wave's searches
+        // cannot wrap it is the coordinate itself, and a scalar branch skips seven vector
+        // instructions (the empty asm keeps the compiler from computing both and selecting).
+        __device__ __forceinline__ float near_origin(int axis, float v) const {
+            if (WRAP && f_.flat_) return v;
+            float x = v;
+            asm volatile("" : "+v"(x));
+            return detail::virtual_coord(x, f_.loc_[axis], f_.width_[axis]);
+        }
         const SpatialFilter& f_;
         uint32_t g_;
         float x_, y_, z_;
@@ -598,17 +633,19 @@ class SpatialFilter {
         }
         // Unit table: a lane whose look-ahead left its unit takes its next non-empty unit
         // (the lowest bit of nm_), with selects, not per-lane branches.  Every unit taken
-        // holds a message, so one take per step is enough; with none left, l_ >= e_ stays.
+        // holds a message, so one take per step is enough; with none left, l_ >= e_ stays
+        // (and the words before the lane's first unit are read, which the table always has,
+        // so the lowest bit needs no select for 0).
         __device__ __forceinline__ void take_unit() {
-            const bool need = l_ >= e_;
-            const uint32_t u = nm_ ? (uint32_t)__builtin_ctz(nm_) : 0u;
-            uint32_t s, e;
+            const bool need = l_ >= e_, left = nm_ != 0u;
+            uint32_t u, s, e;
+            asm("v_ffbl_b32 %0, %1" : "=v"(u) : "v"(nm_));   // ~0 for 0
             read_unit(u, s, e);
-            const bool take = need && nm_ != 0u;
+            const bool take = need && left;
             l_ = take ? s : l_;
             e_ = take ? e : e_;
-            nm_ = need ? (nm_ & (nm_ - 1u)) : nm_;
-            more_ = l_ < e_;
+            nm_ &= nm_ - (need ? 1u : 0u);
+            more_ = !need || left;
         }
         __device__ __forceinline__ void step() {
             ++l_;
@@ -645,6 +682,16 @@ class SpatialFilter {
     __device__ __forceinline__ iterator end() const { return iterator(*this); }
 
  private:
+    // 1 when virtual_coord leaves every candidate of the wave's searches as it is along axis k:
+    // no search reaches the first or last cell.  The messages it visits then lie in the cells
+    // their bins name (positions outside the grid, infinities and NaN are binned into the outer
+    // cells), less than span + 1 cells and a rounding from the origin, which is at most half the
+    // width: half a cell covers the rounding of floor((p - min) / cell) below 2^21 cells.
+    __device__ __forceinline__ bool flat(const detail::SpatialDev& m, int k, int cell) const {
+        const int R = m.span, g = (int)m.grid[k];
+        const bool reach = ((float)R + 1.5f) * m.cell <= 0.5f * m.width[k] && g < (1 << 21);
+        return reach && cell - R >= 1 && cell + R <= g - 2;
+    }
     // Per-lane search origin.  HBM: bins of the grid.  LDS (ebase/xbase/width of the
     // covering group): virtual bin entries, rows of `width` entries for the 9 (3)
     // neighbour rows, x counted from xbase.
@@ -917,7 +964,10 @@ class SpatialFilter {
         } else {
             // one 16-byte load per candidate: the gathers of a wave touch several bins' lines
             // at once, and the texture-address unit pays per line and per load instruction
-            const uint4 r = rec_[l];
+            uint32_t off = l * 16u;
+            asm("" : "+v"(off));
+            const uint4 r = c_.wide ? *reinterpret_cast<const uint4*>(rec_ + (uint64_t)l * 16u)
+                                    : *reinterpret_cast<const uint4*>(rec_ + (uint64_t)off);
             x = __builtin_bit_cast(float, r.x);
             y = __builtin_bit_cast(float, r.y);
             z = DIMS == 3 ? __builtin_bit_cast(float, r.z) : 0.0f;
@@ -940,7 +990,8 @@ class SpatialFilter {
     int m0_, m1_, m2_, s0_, s1_;    // wrapping: last part value and stride per level
     int ebase_, xbase_, ewidth_;    // LDS source: covering group
     const uint32_t* pbm_;
-    const uint4* rec_;              // packed {x, y, z, id} record per message (HBM source)
+    const char* rec_;               // packed 16-byte {x, y, z, id} record per message (HBM source)
+    uint32_t flat_;                 // wrapping: 1 when no search of the wave wraps (wave-uniform)
     uint32_t id_err_;
 };
 
@@ -1603,7 +1654,7 @@ __device__ __forceinline__ __attribute__((address_space(3))) uint32_t* wave_tabl
 // runs agents [first + b * blockDim, ...) of its list.  Shared by the function's own kernel
 // (its launch record in the kernel-argument segment) and the layer kernel (its record in
 // device memory).
-template <typename F>
+template <typename F, bool WIDE = false>
 __device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t x, uint32_t k) {
     const uint32_t first = a.d_first ? load_count(a.d_first) : 0u;
     const uint32_t n = a.d_n ? load_count(a.d_n) : a.n_cap;
@@ -1616,7 +1667,7 @@ __device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t x, 
     uint32_t mn = 0u;
     if constexpr (F::MsgIn::kind == MsgKind::BruteForce) mn = a.d_msg_in_count ? load_count(a.d_msg_in_count) : 0u;
     const ThreadCtx c{a,  ErrState{a.d_error, i}, a.zero_page, a.sink_page, i, a.in_meta, a.env, a.d_step, a.seed, nullptr,
-                      0u, mn,                     o,           a.stream_id, a.unit_tables ? wave_table<F>() : nullptr};
+                      0u, mn,                     o,           a.stream_id, a.unit_tables ? wave_table<F>() : nullptr, WIDE};
     run_agent<F>(c);
 }
 
@@ -1627,9 +1678,23 @@ __global__ void __launch_bounds__(256) agent_function_kernel(const FnArgs a) {
 
 // The same kernel built for 8 resident waves per SIMD (at most 64 VGPRs), for neighbour
 // walks: their loops wait on gathers, and a kernel a few registers above 64 keeps only 7.
+// Its blocks grow to 1024 threads while kMinBigBlocks, two for each of the 256 CUs, remain:
+// 16 waves of neighbouring agents share one L1, whose misses are what a full chip waits on
+// (boids, 1 M: 45.0 M line requests to the L2 with blocks of 256, 36.7 M with 1024).  Boids
+// kernel, blocks of 256 / 512 / 1024: 262,144 agents 128 / 122 / 115 us, 393,216 152 / 142 /
+// 150, 524,288 185 / 174 / 162, 1 M 314 / 303 / 290, 2 M 609 / 611 / 563; of 131,072 and fewer
+// all within 5 %.  Kernels of at most 64 VGPRs read little per candidate and keep 256 (circles,
+// 2 M: 1,184 / 1,194 / 1,249).
+constexpr uint32_t kMinBigBlocks = 512;
 template <typename F>
-__global__ void __launch_bounds__(256, 8) agent_function_kernel_w8(const FnArgs a) {
+__global__ void __launch_bounds__(1024, 8) agent_function_kernel_w8(const FnArgs a) {
     run_function_block<F>(a, blockIdx.x % kXcds, blockIdx.x / kXcds);
+}
+
+// For spatial lists of kWideMessages and more (64-bit message addresses).
+template <typename F>
+__global__ void __launch_bounds__(256) agent_function_kernel_wide(const FnArgs a) {
+    run_function_block<F, true>(a, blockIdx.x % kXcds, blockIdx.x / kXcds);
 }
 
 // Whether a function's launches take agent_function_kernel_w8: when the plain build needs
@@ -1743,7 +1808,7 @@ __global__ void __launch_bounds__(256) layer_kernel(const char* __restrict__ ima
 // seed and error words; each thread runs apt agents, blockDim apart.  A grid
 // smaller than the tile count makes the blocks persistent: logical block b (in
 // XCD-contiguous order) runs tiles [b*T/G, (b+1)*T/G).
-template <typename F>
+template <typename F, bool WIDE>
 __global__ void __launch_bounds__(1024) agent_function_kernel_seg(const FnArgs a, const SegDev* __restrict__ segs,
                                                                   uint32_t nsegs, uint32_t apt) {
     // segs[nsegs] is the sentinel record: its tile_off is the batch's tile count, kept on
@@ -1767,7 +1832,7 @@ __global__ void __launch_bounds__(1024) agent_function_kernel_seg(const FnArgs a
                 const uint32_t i = s.agent_off + local;
                 const ThreadCtx c{a,        ErrState{s.d_error, i}, a.zero_page, a.sink_page, i, s.meta, s.env, s.d_step,
                                   s.seed,   nullptr,                s.msg_off,   s.msg_n,     i,     a.stream_id,
-                                  a.unit_tables ? wave_table<F>() : nullptr};
+                                  a.unit_tables ? wave_table<F>() : nullptr, WIDE};
                 run_agent<F>(c);
             }
         }
@@ -1978,7 +2043,16 @@ void launch_agent_function(const FnArgs& a, uint32_t grid, uint32_t block, uint3
     }
     (void)smem;
     if constexpr (k == MsgKind::Spatial2D || k == MsgKind::Spatial3D) {
+        if (a.wide) {
+            hipLaunchKernelGGL(agent_function_kernel_wide<F>, dim3(grid), dim3(block), fn_lds_bytes<F>(block),
+                               (hipStream_t)stream, a);
+            return;
+        }
         if (block <= 256 && use_w8_kernel<F>()) {
+            while (block < 1024u && grid / 2u >= kMinBigBlocks) {
+                grid = (grid + 1u) / 2u;
+                block *= 2u;
+            }
             hipLaunchKernelGGL(agent_function_kernel_w8<F>, dim3(grid), dim3(block), fn_lds_bytes<F>(block),
                                (hipStream_t)stream, a);
             return;
@@ -1991,8 +2065,15 @@ void launch_agent_function(const FnArgs& a, uint32_t grid, uint32_t block, uint3
 template <typename F>
 void launch_agent_function_seg(const FnArgs& a, const SegDev* segs, uint32_t nsegs, uint32_t apt, uint32_t grid,
                                uint32_t block, void* stream) {
-    hipLaunchKernelGGL(agent_function_kernel_seg<F>, dim3(grid), dim3(block), fn_lds_bytes<F>(block), (hipStream_t)stream,
-                       a, segs, nsegs, apt);
+    if constexpr (reads_spatial<F>()) {
+        if (a.wide) {
+            hipLaunchKernelGGL((agent_function_kernel_seg<F, true>), dim3(grid), dim3(block), fn_lds_bytes<F>(block),
+                               (hipStream_t)stream, a, segs, nsegs, apt);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((agent_function_kernel_seg<F, false>), dim3(grid), dim3(block), fn_lds_bytes<F>(block),
+                       (hipStream_t)stream, a, segs, nsegs, apt);
 }
 
 // Host view of the layer kernel over the functions Fs (see LayerKernel).

@@ -665,6 +665,12 @@ class CUDASimulation {
         unit_tables_ = on;
         clear_graphs();
     }
+    // Neighbour walks address messages with 32-bit offsets in lists below kWideMessages (default)
+    // or with 64-bit addresses in lists of any size.  Results are identical either way.
+    void setWideAddresses(bool on) {
+        wide_ = on;
+        clear_graphs();
+    }
     // The layer kernel of the model's translation unit (set by the model library): layers
     // of several independent functions then run as one launch when in-layer concurrency
     // is on.  setLayerFusion(false) keeps one launch per function, on forked streams.
@@ -935,6 +941,8 @@ class CUDASimulation {
     bool timing_ = false;
     bool stage_enabled_ = false;
     bool unit_tables_ = true;
+    bool wide_ = false;
+    bool wide(const detail::MessageRT& m) const { return wide_ || m.cap >= detail::kWideMessages; }
     detail::LayerKernel layer_kernel_{};
     bool layer_fusion_ = true;
     bool layer_space_warned_ = false;
@@ -1803,6 +1811,7 @@ inline uint32_t CUDASimulation::prepare_function(detail::FnRT& f, void* st, deta
             a.in_meta.wrap_ok = m.wrap_ok;
             a.in_meta.pbm = f.min->pbm;
             a.in_meta.packed = f.min->packed;
+            a.wide = wide(*f.min) ? 1 : 0;
             stage_neighbourhood(f, l, a);
         } else if (f.min->kind == MsgKind::Bucket) {
             a.in_meta.key_min = f.min->key_min;
@@ -1874,7 +1883,7 @@ inline uint32_t CUDASimulation::prepare_function(detail::FnRT& f, void* st, deta
 // In-layer concurrency as one launch: the layer kernel of the model's translation unit
 // runs every function of the layer, each over its own blocks, from launch records held
 // in device memory (fgx_layer_launch).  Layers it cannot take (a function outside the
-// kernel, LDS staging) return false and run on forked streams instead.
+// kernel, LDS staging, 64-bit message addresses) return false and run on forked streams instead.
 inline bool CUDASimulation::launch_layer_fused(const LayerData& layer) {
     if (!layer_fusion_ || !layer_kernel_.kernel || layer.agent_functions.size() > FGX_LAYER_MAX_FNS) return false;
     std::vector<detail::FnRT*> fl;
@@ -1882,7 +1891,7 @@ inline bool CUDASimulation::launch_layer_fused(const LayerData& layer) {
         auto& f = fns_[fn_index_.at(fd.get())];
         if (f.fused_fn == -2) f.fused_fn = layer_kernel_.index_of(f.d->launch);
         if (f.fused_fn < 0) return false;
-        if (stage_enabled_ && f.min && f.min->spatial) return false;
+        if (f.min && f.min->spatial && (stage_enabled_ || wide(*f.min))) return false;
         fl.push_back(&f);
     }
     std::vector<detail::FnArgs> args(fl.size());
@@ -1954,7 +1963,7 @@ inline void CUDASimulation::fill_condition_args(detail::FnRT& f, detail::StateLi
 // three 256-agent blocks resident per CU (52 KB of dynamic LDS each).
 inline void CUDASimulation::stage_neighbourhood(detail::FnRT& f, detail::StateList& l, detail::FnArgs& a) {
     a.stage_ok = 0;
-    if (!stage_enabled_ || f.min->meta.span != 1) return;   // the staged rows cover one bin either side
+    if (!stage_enabled_ || a.wide || f.min->meta.span != 1) return;   // the staged rows cover one bin either side
     const int dims = f.min->meta.dims;
     const char* axes[3] = {"x", "y", "z"};
     for (int k = 0; k < dims; ++k) {

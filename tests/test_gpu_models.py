@@ -83,13 +83,16 @@ def test_boids_bit_exact(n, steps, graphs, staging, tables):
     _compare(sim, ref, 0, "Boid", exact=True)
 
 
-# Lists filled in part (blocks with agents spread over the XCDs), positions on the edges of
-# cells: exact against the oracle.
+# Lists filled in part (blocks with agents spread over the XCDs), blocks of 256, 512 and 1024
+# threads, 32-bit and 64-bit message addresses, searches that cannot wrap and those that can,
+# positions on the edges of cells: exact against the oracle.
 @pytest.mark.parametrize("n,capacity", [(1, 1), (255, 9000), (2047, 2047), (2049, 2049), (2305, 40000), (70001, 300000),
                                         (262161, 262161), (300000, 524800)])
-def test_boids_filled_blocks(n, capacity):
+@pytest.mark.parametrize("wide", [0, 1])
+def test_boids_blocks_and_addresses(n, capacity, wide):
     params, arrs = workloads.boids(capacity, seed=11)
     sim = Simulation("boids_spatial3D", params, seed=11)
+    sim.set_option("wide_addresses", wide)
     sim.set_agents("Boid", arrs)
     arrs = [np.array(a[:n]) for a in arrs]
     for k in range(3):
