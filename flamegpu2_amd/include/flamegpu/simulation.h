@@ -1897,12 +1897,21 @@ inline bool CUDASimulation::launch_layer_fused(const LayerData& layer) {
     std::vector<detail::FnArgs> args(fl.size());
     std::vector<fgx_fn_launch> L(fl.size());
     std::vector<uint32_t> grids(fl.size());
+    for (size_t k = 0; k < fl.size(); ++k) grids[k] = prepare_function(*fl[k], stream_, args[k]);
+    // The blocks start in the order of the functions here (the functions are independent): first
+    // those that read the longer message lists, whose agents take longer, so that the launch
+    // does not end on them with the chip half empty (predator-prey, 1 M prey fleeing 250 k predators and hunted
+    // by them in one layer: 335 us with the prey first, 257 us with the predators first).
+    std::vector<size_t> order(fl.size());
+    for (size_t k = 0; k < fl.size(); ++k) order[k] = k;
+    auto read = [&](size_t k) { return fl[k]->min ? fl[k]->min->cap : 0u; };
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return read(a) > read(b); });
     for (size_t k = 0; k < fl.size(); ++k) {
-        grids[k] = prepare_function(*fl[k], stream_, args[k]);
-        L[k].args = &args[k];
-        L[k].fn = (uint32_t)fl[k]->fused_fn;
-        L[k].blocks = grids[k];
-        L[k].lds_bytes = layer_kernel_.lds_bytes(fl[k]->fused_fn, kFnBlock);
+        const size_t f = order[k];
+        L[k].args = &args[f];
+        L[k].fn = (uint32_t)fl[f]->fused_fn;
+        L[k].blocks = grids[f];
+        L[k].lds_bytes = layer_kernel_.lds_bytes(fl[f]->fused_fn, kFnBlock);
     }
     uint32_t before = 0;
     detail::fgx_check(fgx_layer_space_info(ctx_, &before, nullptr), "layer images");
