@@ -258,6 +258,7 @@ struct FnArgs {
     int32_t wide;                // spatial input: the list may hold kWideMessages or more
     int32_t unit_tables;         // spatial input: build the per-wave unit tables in LDS (0: bin table from HBM)
     uint32_t* d_msg_count_out;   // mandatory output: the launch writes the message count (agent count) here
+    uint32_t* d_launch_count_out;   // or null: the launch writes the count of the agents it runs here
     uint32_t agent_mul, msg_in_mul, msg_out_mul, new_mul, env_mul;
     // neighbourhood staging (spatial message input)
     int32_t stage_ok;                 // agent x/y(/z) present and staged vars chosen

@@ -1661,7 +1661,10 @@ __device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t x, 
     const uint32_t blk = xcd_block(x, k, filled_blocks(n > first ? n - first : 0u));
     if (blk == kNoBlock) return;
     const uint32_t o = blk * blockDim.x + threadIdx.x;
-    if (a.d_msg_count_out && o == 0) *a.d_msg_count_out = n;   // one message per agent (no condition here)
+    if (o == 0) {
+        if (a.d_msg_count_out) *a.d_msg_count_out = n;   // one message per agent (no condition here)
+        if (a.d_launch_count_out) *a.d_launch_count_out = n > first ? n - first : 0u;
+    }
     if (first + o >= n) return;
     const uint32_t i = first + o;
     uint32_t mn = 0u;
@@ -2000,7 +2003,10 @@ __global__ void __launch_bounds__(256) agent_function_kernel_staged(const FnArgs
     const uint32_t blk = xcd_block(filled_blocks(n));
     if (blk == kNoBlock) return;
     const uint32_t b0 = blk * blockDim.x;
-    if (a.d_msg_count_out && b0 == 0 && threadIdx.x == 0) *a.d_msg_count_out = n;
+    if (b0 == 0 && threadIdx.x == 0) {
+        if (a.d_msg_count_out) *a.d_msg_count_out = n;
+        if (a.d_launch_count_out) *a.d_launch_count_out = n;   // (no condition here)
+    }
     if (b0 >= n) return;
     const uint32_t i = b0 + threadIdx.x;
     const bool active = i < n;
