@@ -2120,17 +2120,26 @@ inline void CUDASimulation::enqueue_layer(const LayerData& layer) {
         return;
     }
     // auto spatial sort (CUDASimulation.cu:671-682) and lazy index builds.  Sorts move agent
-    // lists and builds move message lists, so with in-layer concurrency on the builds run on a
-    // stream of their own beside the sorts: both are chains of small latency-bound kernels.
+    // lists and builds move message lists, so with in-layer concurrency on the builds of long
+    // lists run on a stream of their own beside the sorts.  The fork and the join take 18 us, more
+    // than the chains of short lists save (20 steps: predator-prey with 20 k prey 9.7 ms side by
+    // side, 9.0 in turn; 65,536 boids 3.59 / 3.53; 131,072 circles the same; 262,144 boids
+    // 4.33 / 4.41; predator-prey with 1 M prey, 10 steps, 9.6 / 10.0).
+    constexpr uint32_t kOverlapAgents = 1u << 17;
     bool sorts = false, builds = false;
+    uint32_t longest = 0;
     for (auto& fd : layer.agent_functions) {
         auto& f = fns_[fn_index_.at(fd.get())];
         const unsigned period = f.d->parent->sortPeriod;
-        sorts = sorts || (f.sort_dims && period && step_ % period == 0);
-        builds = builds || (f.min && f.min->pbm_dirty &&
-                            (f.min->spatial || f.min->kind == MsgKind::Bucket || is_array_kind(f.min->kind)));
+        const bool sort = f.sort_dims && period && step_ % period == 0;
+        const bool build = f.min && f.min->pbm_dirty &&
+                           (f.min->spatial || f.min->kind == MsgKind::Bucket || is_array_kind(f.min->kind));
+        sorts = sorts || sort;
+        builds = builds || build;
+        if (sort) longest = std::max(longest, f.agent->states.at(f.in_state).cap);
+        if (build) longest = std::max(longest, f.min->cap);
     }
-    const bool overlap = sorts && builds && cuda_config_.inLayerConcurrency && !timing_;
+    const bool overlap = sorts && builds && longest >= kOverlapAgents && cuda_config_.inLayerConcurrency && !timing_;
     void* bst = stream_;
     if (overlap) {
         if (!build_stream_) detail::fgx_check(fgx_stream_create(&build_stream_), "stream create");
