@@ -26,7 +26,7 @@ struct BucketArgs {
     KeyArgs ka;
     const uint32_t* d_n;
     uint32_t n_cap;
-    uint32_t shift, buckets, tiles, bins;
+    uint32_t shift, buckets, tiles, tile, bins;   // tile: elements a tile
     const float* x;
     const float* y;
     const float* z;
@@ -129,13 +129,24 @@ __device__ __forceinline__ void zero_rows(uint16_t* rows, uint32_t n) {
     for (uint32_t k = threadIdx.x; k < (n + 1u) / 2u; k += BT) reinterpret_cast<uint32_t*>(rows)[k] = 0u;
 }
 
+// The tiles of `size` elements that hold elements (at least one): only these are counted, summed
+// and split, on all XCDs, whatever the capacity the launches are sized for (predator-prey, 1 M
+// prey in lists about 40 % full, a launch on average: count 11.3 -> 7.4 us, prefix 7.8 -> 5.8,
+// split 27.4 -> 15.6).
+__device__ __forceinline__ uint32_t filled_tiles(uint32_t n, uint32_t size) {
+    const uint32_t f = (__builtin_amdgcn_readfirstlane(n) + size - 1u) / size;
+    return f ? f : 1u;
+}
+
 // ---------------------------------------------------------------- count
 template <uint32_t BT, uint32_t ITEMS>
 __global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
     __shared__ uint32_t s_hist[kMaxBuckets];
     __shared__ uint32_t s_met;
-    const uint32_t tile = xcd_block(), t = threadIdx.x;
+    const uint32_t t = threadIdx.x;
     const uint32_t n = load_count(a.d_n, a.n_cap);
+    const uint32_t tile = xcd_filled_block(filled_tiles(n, BT * ITEMS));
+    if (tile == kNoBlock) return;
     for (uint32_t b = t; b < a.buckets; b += BT) s_hist[b] = 0u;
     if (t == 0) s_met = 0u;
     __syncthreads();
@@ -173,8 +184,9 @@ __global__ void __launch_bounds__(1024) k_bucket_prefix(BucketArgs a) {
     __shared__ uint32_t s_red[16];
     const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
     const uint32_t b = blockIdx.x * 64u + lane;
-    const uint32_t per = (a.tiles + 15u) / 16u;
-    const uint32_t t0 = w * per < a.tiles ? w * per : a.tiles, t1 = t0 + per < a.tiles ? t0 + per : a.tiles;
+    const uint32_t tiles = filled_tiles(load_count(a.d_n, a.n_cap), a.tile);
+    const uint32_t per = (tiles + 15u) / 16u;
+    const uint32_t t0 = w * per < tiles ? w * per : tiles, t1 = t0 + per < tiles ? t0 + per : tiles;
     const bool on = b < a.buckets;
     uint32_t sum = 0;
     for (uint32_t t = t0; t < t1; t += 8u) {
@@ -206,7 +218,7 @@ __global__ void __launch_bounds__(1024) k_bucket_prefix(BucketArgs a) {
     if (blockIdx.x == 0) {
         uint32_t met = 0, all = 0;
         if (a.stage_above)
-            for (uint32_t t = threadIdx.x; t < a.tiles; t += 1024u) met += a.met[t];
+            for (uint32_t t = threadIdx.x; t < tiles; t += 1024u) met += a.met[t];
         block_prefix<16>(met, s_red, &all);
         if (threadIdx.x == 0) *a.stage = a.stage_above && all > a.stage_above ? 1u : 0u;
     }
@@ -228,10 +240,11 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
     __shared__ uint32_t s_key[T];
     __shared__ uint16_t s_loc[T];
     __shared__ uint32_t s_red[W];
-    const uint32_t tile = xcd_block(), t = threadIdx.x, w = t >> 6, lane = lane_id();
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
     const uint32_t n = load_count(a.d_n, a.n_cap), nb = a.buckets;
+    const uint32_t tile = xcd_filled_block(filled_tiles(n, T));
+    if (tile == kNoBlock) return;
     const uint32_t base = tile * T;
-    if (base >= n && tile != 0) return;
     const uint32_t cnt = base < n ? (n - base < T ? n - base : T) : 0u;
     // this thread's buckets: their totals and the tile's offsets are loaded beside the positions
     constexpr uint32_t Q = MAXB / BT;
@@ -739,6 +752,7 @@ int bucket_sort(const BucketPlan& p, const KeyArgs& ka, uint32_t bins, const uin
     a.shift = p.shift;
     a.buckets = p.buckets;
     a.tiles = p.tiles;
+    a.tile = p.threads * p.items;
     a.bins = bins;
     a.x = x;
     a.y = y;

@@ -112,6 +112,15 @@ __device__ __forceinline__ uint32_t xcd_block() {
     return x * q + (x < r ? x : r) + k;
 }
 
+// The same over the first `filled` blocks only (at most the grid's), kNoBlock for the others:
+// a launch sized for a list's capacity runs the blocks with elements on all XCDs.
+constexpr uint32_t kNoBlock = 0xFFFFFFFFu;
+__device__ __forceinline__ uint32_t xcd_filled_block(uint32_t filled) {
+    constexpr uint32_t kXcds = 8;
+    const uint32_t x = blockIdx.x % kXcds, k = blockIdx.x / kXcds, q = filled / kXcds, r = filled % kXcds;
+    return k < q + (x < r ? 1u : 0u) ? x * q + (x < r ? x : r) + k : kNoBlock;
+}
+
 // ---------------------------------------------------------------- wave64 helpers
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 

@@ -727,6 +727,14 @@ def test_index_sizes_and_shapes(ctx, what, dims, n, axis, positions, use_dn):
     _index_case(ctx, what, dims, n, axis, positions, by, use_dn)
 
 
+# Lists filled in part: fewer tiles with elements than XCDs, whole tiles, one element more.
+@pytest.mark.parametrize("what,dims,n,axis,filled", [
+    ("messages", 3, 100003, 30, 1024), ("agents", 3, 100003, 30, 7 * 1024), ("messages", 2, 100003, 60, 9 * 1024 + 1),
+    ("messages", 3, 600000, 40, 1), ("agents", 3, 600000, 40, 4096 * 17 + 1), ("messages", 2, 3200001, 400, 16384 * 3)])
+def test_index_filled_tiles(ctx, what, dims, n, axis, filled):
+    _index_case(ctx, what, dims, n, axis, _uniform, [4, 8, 1], filled)
+
+
 @pytest.mark.parametrize("n", [1, 1023, 1025, 200 * 1024, 200 * 1024 + 1, 8 * 200 * 1024 - 1, 8 * 200 * 1024 + 3])
 def test_reduce_stats_block_edges(ctx, n):
     # sizes around the blocks and batches of the one-pass statistics, on values far from zero
