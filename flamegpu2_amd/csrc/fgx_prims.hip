@@ -1,11 +1,12 @@
 // libfgx: hot-path primitives for gfx950 (wave64).
 //
-//   message-list build : bin key + run-aggregated wave64 histogram -> exclusive scan in
-//                        passes ordered by kernel boundaries (tile sums, then tile
-//                        prefixes) -> bin start table -> index scatter (bins grouped) ->
-//                        in-bin order restored by index (large bins sorted by one block
-//                        each) -> SoA payload scatter
-//   agent spatial sort : same pipeline with the unclamped sort key
+//   message-list build : fgx_bucket_sort.hip, but for sparse bin tables, segmented lists and
+//                        more than 12 M elements: bin key + run-aggregated wave64 histogram
+//                        -> exclusive scan in passes ordered by kernel boundaries (tile sums,
+//                        then tile prefixes) -> bin start table -> index scatter (bins
+//                        grouped) -> in-bin order restored by index (large bins sorted by
+//                        one block each) -> SoA payload scatter
+//   agent spatial sort : the same, with the unclamped sort key
 //   compaction/births  : kept count per tile, then per-tile prefixes, ballot ranks and
 //                        the copy of every variable (two passes, no inter-block waits)
 //   reduction          : fixed-shape (deterministic) tree
