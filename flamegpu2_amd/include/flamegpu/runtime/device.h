@@ -444,7 +444,7 @@ constexpr uint32_t kHashId = name_hash("id", 3);
 // Over large lists the walk is bound by vector issue (boids, 1 M: 211 M wave instructions,
 // 118 a candidate, 343 us): scalar bases with 32-bit lane offsets (load_msg_var, fetch),
 // virtual coordinates only where a search can wrap (near_origin) and a shorter unit step
-// (take_unit) leave 176 M (95 a candidate) and, with blocks of 1024, 290 us.
+// (take_unit) leave 165 M (92 a candidate) and, with blocks of 1024, 290 us.
 //
 // Source: the message list in HBM (bin table pbm, packed records), or, in the staged
 // kernel when every lane of the wave is covered by the block's LDS copy, the LDS tables
