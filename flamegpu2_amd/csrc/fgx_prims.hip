@@ -1156,7 +1156,9 @@ static int run_bin_sort(fgx_ctx* ctx, const KeyArgs& ka, uint32_t bins, uint64_t
     const bool capturing = cap != hipStreamCaptureStatusNone;
     //
     // The bucket sort works in the key arrays only and leaves the histogram region of its own
-    // bin count as it found it.
+    // bin count as it found it: neither cleared nor dirtied.  It therefore never stands for the
+    // first sort of the rule above (a later sort of the buffer through global atomics, of the
+    // same bin count but another size, clears), and counts as one of another bin count.
     bool clean = false;
     const bool record = ctx && ctx->c.keep_zero && !shared_space;
     BucketPlan plan;
@@ -1170,8 +1172,11 @@ static int run_bin_sort(fgx_ctx* ctx, const KeyArgs& ka, uint32_t bins, uint64_t
         clean = capturing ? single : zero;
         if (it != clean_record().end()) clean_record().erase(it);   // re-recorded once every launch is enqueued
         if (buckets && zero && !capturing) clean_record()[scratch] = bins;
-        if (hit == bins_history().end()) bins_history()[scratch] = bins;
-        else if (hit->second != bins) hit->second = kMixedBins;
+        if (hit != bins_history().end()) {
+            if (hit->second != bins) hit->second = kMixedBins;
+        } else if (!buckets) {
+            bins_history()[scratch] = bins;
+        }
     }
     if (buckets) return bucket_sort(plan, ka, bins, d_n, n_cap, x, y, z, vt, starts_read ? start_out : nullptr, key, sub, tmp, st);
     int rc = FGX_OK;

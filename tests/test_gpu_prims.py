@@ -473,6 +473,51 @@ def test_spatial_build_captured_on_fresh_scratch():
     c.close()
 
 
+def test_captured_sorts_of_both_kinds_share_scratch():
+    """One zero-kept scratch buffer, captured as its first uses: a build sorted through LDS, one
+    of the same 128^3 bins sorted through global atomics (fewer elements, too many bins for
+    LDS), one of 10^3 bins whose key arrays lie over the first two's histogram.  The second
+    must carry its own clearing launch: every replay equals the oracle."""
+    from flamegpu2_amd import fgx
+    c = fgx.Context(0)
+    c.set_option(fgx.FGX_OPT_KEEP_SCRATCH_ZERO, 1)
+    rng = np.random.default_rng(29)
+    builds = []
+    for n, radius in [(300000, 0.025), (200000, 0.025), (200000, 0.32)]:
+        box = ([0.0] * 3, [3.2] * 3, radius)
+        m = fgx.spatial_meta(3, *box)
+        P = rng.uniform(0, 3.2, size=(3, n)).astype(np.float32)
+        pbm_o, _, outs_o = O.spatial_build(O.spatial_meta(3, *box), P[0], P[1], P[2])
+        builds.append((m, n, [dev(p) for p in P], [empty(n, np.float32) for _ in range(3)], empty(m.bins + 1, np.uint32),
+                       pbm_o, outs_o))
+    assert builds[0][0].bins == builds[1][0].bins == 128 ** 3 and builds[2][0].bins == 1000
+    sb = max(fgx.scratch_bytes(fgx.FGX_OP_SPATIAL_BUILD, n, m.bins) for m, n, *_ in builds)
+    s = scratch(sb)
+    st = fgx.stream_create()
+
+    def enqueue():
+        for m, n, d_in, d_out, pbm, _, _ in builds:
+            x = [ptr(t) for t in d_in]
+            fgx.spatial_build(c, m, n, *x, x, [ptr(t) for t in d_out], [4, 4, 4], ptr(pbm), ptr(s), sb, stream=st)
+
+    g = fgx.graph_capture(st, enqueue)
+    try:
+        for _ in range(3):
+            fgx.graph_launch(g, st)
+            fgx.stream_synchronize(st)
+            for m, n, _, d_out, pbm, pbm_o, outs_o in builds:
+                assert np.array_equal(host(pbm, np.uint32, m.bins + 1), pbm_o)
+                for a in range(3):
+                    assert np.array_equal(host(d_out[a], np.float32, n), outs_o[a])
+                for t in d_out + [pbm]:
+                    fgx.fill_u32(ptr(t), 0, t.alloc_bytes // 4)   # so that each check sees fresh output
+            sync()
+    finally:
+        fgx.graph_destroy(g)
+        fgx.stream_destroy(st)
+    c.close()
+
+
 def test_spatial_build_large_bin_table(ctx):
     # 4.1 M bins (> 1,024 scan tiles): the bin counts go through the block-scanned path
     _build_case(ctx, 3, 1 << 20, 16.0, 0.1, 21)
