@@ -252,7 +252,9 @@ class BatchSimulation {
     void after_launch(FnB& f);
     void enqueue_step();
     void launch(FnB& f);
+    // Steps are enqueued and not waited for: a graph may still be running when it is dropped.
     void clear_graphs() {
+        if (!graphs_.empty()) fgx_stream_synchronize(stream_);
         for (auto& g : graphs_) fgx_graph_destroy(g.g);
         graphs_.clear();
     }

@@ -925,7 +925,9 @@ class CUDASimulation {
         std::unique_ptr<AgentVector> v;
     };
     std::map<detail::StateList*, HostNew> host_new_;   // pending host-created agents, by state list
+    // Steps are enqueued and not waited for: a graph may still be running when it is dropped.
     void clear_graphs() {
+        if (!graphs_.empty()) fgx_stream_synchronize(stream_);
         for (auto& g : graphs_) fgx_graph_destroy(g.g);
         graphs_.clear();
     }
@@ -2401,6 +2403,7 @@ inline bool CUDASimulation::step() {
                              kMaxStepGraphs);
                 graph_evict_warned_ = true;
             }
+            synchronize();   // the graph may still be running
             fgx_graph_destroy(graphs_[lru].g);
             graphs_.erase(graphs_.begin() + (std::ptrdiff_t)lru);
         }

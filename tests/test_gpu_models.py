@@ -146,6 +146,38 @@ def test_predprey_full_config_three_steps():
     _compare(sim, ref, 1, "Predator", exact=True)
 
 
+def test_graphs_dropped_while_steps_run():
+    """Options that drop the step graphs, set with steps enqueued and not waited for."""
+    n = 200000
+    params, arrs = workloads.boids(n, seed=19)
+    sim = Simulation("boids_spatial3D", params, seed=19)
+    sim.set_agents("Boid", arrs)
+    ref = O.Sim(1, params, 19)
+    ref.set_agents(0, arrs)
+    for key, value in [("unit_tables", 0), ("unit_tables", 1), ("wide_addresses", 1), ("wide_addresses", 0)]:
+        sim.step(2)
+        sim.set_option(key, value)
+    sim.step(2)
+    ref.step(10)
+    _compare(sim, ref, 0, "Boid", exact=True)
+    # the same in a batch, and against the same simulation alone
+    from flamegpu2_amd.models import Batch
+    b = Batch("circles_spatial3D", workloads.circles(20000, seed=5)[0])
+    params, arrs = workloads.circles(20000, seed=5)
+    h = b.add(params, 5, 100, {"Circle": arrs})
+    alone = Simulation("circles_spatial3D", params, seed=5)
+    alone.set_agents("Circle", arrs)
+    for value in (0, 1):
+        b.step(5)   # graphs from the third step of a stable batch
+        b.set_option("unit_tables", value)
+    b.step(5)
+    alone.step(15)
+    got, exp = b.get_agents(h, "Circle"), alone.get_agents("Circle")
+    assert np.array_equal(got[1], exp[1])
+    for x, y in zip(got[0], exp[0]):
+        assert np.array_equal(x, y)
+
+
 def test_graph_and_eager_agree():
     params, arrs = workloads.boids(20000, seed=9)
     a = Simulation("boids_spatial3D", params, seed=9)
