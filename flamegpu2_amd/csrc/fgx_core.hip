@@ -340,6 +340,12 @@ int fgx_ctx_set_option(fgx_ctx* ctx, int option, int value) {
     return FGX_OK;
 }
 
+int fgx_sort_clears(fgx_ctx* ctx, uint64_t* n) {
+    if (!ctx || !n) return fail(FGX_ERR_ARG, "fgx_sort_clears: NULL context or result");
+    *n = ctx->c.sort_clears;
+    return FGX_OK;
+}
+
 int fgx_device_info(fgx_ctx* ctx, int* cu_count, int* xcd_count, size_t* hbm_bytes) {
     if (!ctx) return fail(FGX_ERR_ARG, "fgx_device_info: NULL context");
     if (cu_count) *cu_count = ctx->c.cu_count;

@@ -37,6 +37,7 @@ struct Ctx {
     size_t hbm_bytes = 0;
     // FGX_OPT_KEEP_SCRATCH_ZERO: bin sorts leave their histogram zeroed
     int keep_zero = 0;
+    uint64_t sort_clears = 0;   // histogram clearing launches that bin sorts have enqueued
     LayerSpace layers;
 };
 

@@ -1183,6 +1183,7 @@ static int run_bin_sort(fgx_ctx* ctx, const KeyArgs& ka, uint32_t bins, uint64_t
     if (!clean) {
         rc = fgx_fill_u32(hist, 0u, (size_t)bins + 2, stream);
         if (rc) return rc;
+        if (ctx) ++ctx->c.sort_clears;
     }
     const uint32_t g = stream_grid(ctx ? &ctx->c : nullptr, n_cap);
     if (n_cap) {

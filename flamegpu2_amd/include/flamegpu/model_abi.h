@@ -341,6 +341,7 @@ FGXM_EXPORT int fgxm_stat(fgxm_sim* s, const char* key, uint64_t* out) {
     return fgxm_detail::guard([&] {
         const std::string k = key ? key : "";
         if (k == "fused_layer_launches") *out = s->sim->fusedLayerLaunches();
+        else if (k == "graph_captures") *out = s->sim->graphCaptures();
         else if (k == "layer_images") *out = s->sim->layerImages();
         else throw flamegpu::exception::InvalidArgument("unknown counter " + k);
     });

@@ -683,6 +683,8 @@ class CUDASimulation {
         layer_fusion_ = on;
         clear_graphs();
     }
+    // Step graphs captured so far.
+    uint64_t graphCaptures() const { return graph_captures_; }
     // Fused layer launches enqueued so far (graph replays not counted).
     uint64_t fusedLayerLaunches() const { return fused_launches_; }
     uint64_t layerImages() {
@@ -791,7 +793,7 @@ class CUDASimulation {
         void* p = nullptr;
         alloc(&p, *bytes);
         detail::fgx_check(fgx_scratch_clear(p, *bytes, stream_), "scratch clear");
-        sorted_scratch_.erase(p);
+        cleared_scratch_.erase(p);
         return p;
     }
     void grow_list(detail::StateList& l, uint32_t cap);
@@ -906,7 +908,7 @@ class CUDASimulation {
     struct GraphEntry {
         std::vector<void*> start, end;
         std::vector<uint8_t> swaps;   // the step's transition plan (which transitions swap lists)
-        bool stale = false;           // recorded a layer image upload: captured again next time
+        bool stale = false;           // recorded a layer image upload or a first clearing launch: captured again next time
         bool concurrent = true;       // captured with in-layer concurrency on
         fgx_graph* g = nullptr;
         uint64_t last_use = 0;
@@ -917,6 +919,7 @@ class CUDASimulation {
     static constexpr size_t kMaxStepGraphs = 8;
     std::vector<GraphEntry> graphs_;
     uint64_t graph_uses_ = 0;
+    uint64_t graph_captures_ = 0;
     bool graph_evict_warned_ = false;
     bool graph_eligible_ = false;
     bool populations_set_ = false;   // setPopulationData since the last step: re-check capacities
@@ -949,12 +952,17 @@ class CUDASimulation {
     bool layer_fusion_ = true;
     bool layer_space_warned_ = false;
     bool new_layer_images_ = false;   // the enqueue being captured uploaded a layer image
-    // sort scratch buffers that a sort has used: a capture that holds a buffer's first sort
+    // sort scratch buffers whose first clearing sort has been enqueued: a capture that holds one
     // also holds its clearing launch, so the graph is captured again after one run
-    std::unordered_set<const void*> sorted_scratch_;
-    bool first_sorts_ = false;        // the enqueue being captured holds a buffer's first sort
+    std::unordered_set<const void*> cleared_scratch_;
+    uint64_t sort_clears_ = 0;        // clearing launches enqueued so far (fgx_sort_clears)
+    bool first_clears_ = false;       // the enqueue being captured holds a buffer's first clearing launch
+    // Called after each sort or build on `scratch`.
     void note_sort(const void* scratch) {
-        if (sorted_scratch_.insert(scratch).second) first_sorts_ = true;
+        uint64_t n = 0;
+        detail::fgx_check(fgx_sort_clears(ctx_, &n), "sort clears");
+        if (n != sort_clears_ && cleared_scratch_.insert(scratch).second) first_clears_ = true;
+        sort_clears_ = n;
     }
     uint64_t fused_launches_ = 0;
     float bin_mult_ = 1.0f;
@@ -2164,13 +2172,13 @@ inline void CUDASimulation::enqueue_layer(const LayerData& layer) {
                 by.push_back(v.bytes);
             }
             tick("sort:" + f.agent->d->name, stream_, true);
-            note_sort(l.sort_scratch);
             detail::fgx_check(fgx_agent_sort(ctx_, f.sort_dims, f.min->meta.min, f.min->meta.max, f.min->meta.radius, l.d_count,
                                              l.cap, (const float*)l.vars[ix].cur, (const float*)l.vars[iy].cur,
                                              f.sort_dims == 3 ? (const float*)l.vars[iz].cur : nullptr,
                                              (uint32_t)l.vars.size(), src.data(), dst.data(), by.data(), l.sort_scratch,
                                              l.sort_scratch_bytes, stream_),
                               "agent spatial sort");
+            note_sort(l.sort_scratch);
             tick("sort:" + f.agent->d->name, stream_, false);
             for (auto& v : l.vars) std::swap(v.cur, v.alt);
         }
@@ -2189,7 +2197,6 @@ inline void CUDASimulation::enqueue_layer(const LayerData& layer) {
                 by.push_back(v.bytes);
             }
             tick("build:" + m.d->name, bst, true);
-            note_sort(m.build_scratch);
             // the walk's {x, y, z, id} records are written by the build's scatter
             const int ii = m.var_index("id");
             const int32_t rec_vars[4] = {ix, iy, m.meta.dims == 3 ? iz : -1,
@@ -2201,6 +2208,7 @@ inline void CUDASimulation::enqueue_layer(const LayerData& layer) {
                                                         rec_vars, m.packed, m.pbm, m.build_scratch,
                                                         m.build_scratch_bytes, bst),
                               "message index build");
+            note_sort(m.build_scratch);
             for (auto& v : m.vars) std::swap(v.cur, v.alt);
             tick("build:" + m.d->name, bst, false);
             m.pbm_dirty = false;
@@ -2217,11 +2225,11 @@ inline void CUDASimulation::enqueue_layer(const LayerData& layer) {
             tick("build:" + m.d->name, bst, true);
             if (m.kind == MsgKind::Bucket) {
                 const int ik = m.var_index("_key");
-                note_sort(m.build_scratch);
                 detail::fgx_check(fgx_bucket_build(ctx_, m.key_min, m.keys, m.d_count, m.cap, (const int32_t*)m.vars[ik].cur,
                                                    (uint32_t)m.vars.size(), src.data(), dst.data(), by.data(), m.pbm,
                                                    m.build_scratch, m.build_scratch_bytes, bst),
                                   "bucket message index build");
+                note_sort(m.build_scratch);
             } else {
                 const int ii = m.var_index("___INDEX");
                 detail::fgx_check(fgx_array_build(ctx_, m.length, m.d_count, m.cap, (const uint32_t*)m.vars[ii].cur,
@@ -2413,11 +2421,12 @@ inline bool CUDASimulation::step() {
             e.swaps = swaps;
             e.concurrent = cuda_config_.inLayerConcurrency;
             new_layer_images_ = false;
-            first_sorts_ = false;
+            first_clears_ = false;
             detail::fgx_check(fgx_graph_begin(stream_), "graph begin");
             enqueue_step();
             detail::fgx_check(fgx_graph_end(stream_, &e.g), "graph end");
-            e.stale = new_layer_images_ || first_sorts_;
+            ++graph_captures_;
+            e.stale = new_layer_images_ || first_clears_;
             e.end = buffer_state();
             set_buffer_state(start);   // capture recorded the work; nothing has run yet
             graphs_.push_back(std::move(e));

@@ -63,6 +63,9 @@ int fgx_device_info(fgx_ctx* ctx, int* cu_count, int* xcd_count, size_t* hbm_byt
  * and capture again after changing it). */
 enum { FGX_OPT_KEEP_SCRATCH_ZERO = 1 };
 int fgx_ctx_set_option(fgx_ctx* ctx, int option, int value);
+/* Histogram clearing launches that bin sorts on this context have enqueued so far (sorts
+ * through LDS need none): a capture during which it grew replays them. */
+int fgx_sort_clears(fgx_ctx* ctx, uint64_t* n);
 
 /* ---------------------------------------------------------------- memory, streams, events, graphs
  * Thin wrappers so the C++ runtime never includes HIP headers. */

@@ -60,7 +60,7 @@ int fgxm_kernel_times(fgxm_sim* sim, char* buf, uint32_t buflen, int reset);
 int fgxm_timed_steps(fgxm_sim* sim, uint32_t steps, double* ms);
 int fgxm_step_counter(fgxm_sim* sim, uint32_t* out);
 /* Runtime counters (no counterpart in the reference): "fused_layer_launches" (layers
- * enqueued as one launch, graph replays not counted), "layer_images" (fused-layer images
+ * enqueued as one launch, graph replays not counted), "graph_captures" (step graphs captured), "layer_images" (fused-layer images
  * the simulation's context holds). */
 int fgxm_stat(fgxm_sim* sim, const char* key, uint64_t* out);
 /* CUDAEnsemble::simulate (src/flamegpu/simulation/CUDAEnsemble.cu) over `nplans` runs of

@@ -146,6 +146,23 @@ def test_predprey_full_config_three_steps():
     _compare(sim, ref, 1, "Predator", exact=True)
 
 
+# A simulation's agent list swaps buffers once a step: two arrangements, one graph each.  Sorts
+# through LDS (3,000 and 50,000 agents over 64^3 bins or fewer) clear no histogram; the sparse
+# table (2,000 agents over 128^3 bins) takes the sort through global atomics, whose first graph
+# holds the clearing launches and is captured again after one run.
+@pytest.mark.parametrize("n,width,captures", [(3000, 0.45, 2), (50000, 1.2, 2), (2000, 6.4, 3)])
+def test_step_graph_captures(n, width, captures):
+    params, arrs = workloads.boids(n, seed=31, width=width)
+    sim = Simulation("boids_spatial3D", params, seed=31)
+    sim.set_agents("Boid", arrs)
+    ref = O.Sim(1, params, 31)
+    ref.set_agents(0, arrs)
+    sim.step(6)
+    ref.step(6)
+    assert sim.stat("graph_captures") == captures
+    _compare(sim, ref, 0, "Boid", exact=True)
+
+
 def test_graphs_dropped_while_steps_run():
     """Options that drop the step graphs, set with steps enqueued and not waited for."""
     n = 200000
