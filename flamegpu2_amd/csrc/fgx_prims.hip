@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 namespace fgx {
 
@@ -902,7 +903,7 @@ __device__ __forceinline__ StatSet<Acc> merge_stats(const StatSet<Acc>& a, const
     r.dev = a.dev + b.dev;
     if (a.n > 0.0 && b.n > 0.0) {
         const double d = b.shifted / b.n - a.shifted / a.n;
-        r.dev += d * d * (a.n * (b.n / r.n));
+        r.dev += d * (d * (a.n * (b.n / r.n)));   // d * d may overflow where the product does not
     }
     return r;
 }
@@ -1003,6 +1004,17 @@ __global__ void __launch_bounds__(kStatBlock) k_stats_partial(const T* __restric
     }
 }
 
+// The squared deviations of doubles from sum / n where sums or differences leave the range of
+// the type.  A sum that overflowed is infinitely far from every finite value, an infinity is
+// no distance from an infinite mean (NaN); with a finite mean a NaN can only come from
+// differences beyond the range, whose squares are infinite.  (When sum / n is finite and so
+// are all squared differences from it, those from the list's first value stay in range too.)
+__device__ __forceinline__ double deviations_in_range(const StatSet<double>& a) {
+    if (__builtin_isnan(a.sum)) return a.sum;
+    if (__builtin_isinf(a.sum)) return __builtin_isinf(a.mn) || __builtin_isinf(a.mx) ? __builtin_nan("") : __builtin_inf();
+    return __builtin_isnan(a.dev) ? __builtin_inf() : a.dev;
+}
+
 // out[0] sum, out[1] min, out[2] max (as Acc), out[3] the sum of squared deviations from
 // the mean (0 when n == 0), as the reference's standard deviation takes it
 // (include/flamegpu/simulation/AgentLoggingConfig.h, getAgentVariableStandardDevFunc;
@@ -1031,6 +1043,7 @@ __global__ void __launch_bounds__(kBlock) k_stats_final(const Acc* __restrict__ 
         out[0] = a.sum;
         out[1] = a.mn;
         out[2] = a.mx;
+        if constexpr (std::is_same<Acc, double>::value) a.dev = deviations_in_range(a);
         reinterpret_cast<double*>(out)[3] = a.dev;
     }
 }

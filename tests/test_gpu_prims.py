@@ -780,6 +780,30 @@ def test_index_filled_tiles(ctx, what, dims, n, axis, filled):
     _index_case(ctx, what, dims, n, axis, _uniform, [4, 8, 1], filled)
 
 
+# Doubles whose spread nears or leaves the type's range, and infinities and NaN: the squared
+# deviations are those of (x - sum / n)^2 in double precision, finite, infinite or NaN alike.
+@pytest.mark.parametrize("values", [
+    [1e308, -1e308], [1e308, -1e308, 3.0, -5.0], [1.5e308, 1.5e308], [-1.5e308] * 3, [0.9e154, -0.9e154],
+    [1e300, 2.0, -1e300], [np.inf, 1.0], [1.0, np.inf], [np.inf, -np.inf], [np.nan, 1.0], [1.0, 2.0, np.nan], [7e307] * 2, [5.0]])
+@pytest.mark.parametrize("repeat", [1, 700])
+def test_reduce_stats_extremes(ctx, values, repeat):
+    from flamegpu2_amd import fgx
+    a = np.tile(np.array(values, np.float64), repeat)
+    sb = fgx.scratch_bytes(fgx.FGX_OP_STATS, 0)
+    s, o = scratch(sb), empty(4, np.float64)
+    fgx.reduce_stats(ctx, 1, ptr(dev(a)), len(a), ptr(o), ptr(s), sb)
+    sync()
+    sm, mn, mx, sq = host(o, np.float64, 4)
+    if not np.isnan(a).any():
+        assert mn == a.min() and mx == a.max()
+    with np.errstate(all="ignore"):
+        ref = ((a - sm / len(a)) ** 2).sum()   # about the sum that was returned: its order is open
+    if np.isfinite(ref):
+        assert abs(sq - ref) <= 1e-12 * ref
+    else:
+        assert np.isnan(sq) if np.isnan(ref) else sq == ref
+
+
 @pytest.mark.parametrize("n", [1, 1023, 1025, 200 * 1024, 200 * 1024 + 1, 8 * 200 * 1024 - 1, 8 * 200 * 1024 + 3])
 def test_reduce_stats_block_edges(ctx, n):
     # sizes around the blocks and batches of the one-pass statistics, on values far from zero
