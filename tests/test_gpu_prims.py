@@ -823,3 +823,36 @@ def test_reduce_stats_block_edges(ctx, n):
     assert mn == a.min() and mx == a.max()
     assert abs(sm - float(x.sum())) <= 1e-13 * float(x.sum())
     assert abs(sq - float(ref)) <= 1e-13 * float(ref) + 1e-300
+
+
+# The other types at the same sizes.  Integer sums, minima and maxima are exact.  Deviations:
+# values of at most 2^40 and their differences from the first are exact in a double, and means
+# and merges round as above: 1e-13.
+@pytest.mark.parametrize("code,dtype", [(0, np.float32), (2, np.int32), (3, np.uint32), (4, np.int64), (5, np.uint64)])
+@pytest.mark.parametrize("n", [1, 63, 1023, 1025, 200 * 1024, 200 * 1024 + 1, 8 * 200 * 1024 - 1, 8 * 200 * 1024 + 3])
+def test_reduce_stats_block_edges_types(ctx, code, dtype, n):
+    from flamegpu2_amd import fgx
+    rng = np.random.default_rng(n + code)
+    if dtype == np.float32:
+        a = (1.0e4 + rng.normal(size=n)).astype(dtype)
+    else:
+        i = np.iinfo(dtype)
+        wide = np.dtype(dtype).itemsize == 8
+        lo, hi = (-(1 << 40) if i.min else 0, 1 << 40) if wide else (i.min, i.max)
+        a = rng.integers(lo, hi, size=n, dtype=dtype, endpoint=True)
+        a[n // 2], a[-1] = lo, hi
+    sb = fgx.scratch_bytes(fgx.FGX_OP_STATS, 0)
+    s, o = scratch(sb), empty(4, np.float64)
+    fgx.reduce_stats(ctx, code, ptr(dev(a)), n, ptr(o), ptr(s), sb)
+    sync()
+    raw = host(o, np.float64, 4)
+    x = a.astype(np.longdouble)
+    if dtype == np.float32:
+        assert raw[1] == float(a.min()) and raw[2] == float(a.max())
+        assert abs(raw[0] - float(x.sum())) <= 1e-13 * abs(float(x.sum()))
+    else:
+        got = raw.view(np.int64 if np.iinfo(dtype).min else np.uint64)
+        assert int(got[0]) == sum(int(v) for v in np.add.reduceat(a.astype(got.dtype), np.arange(0, n, 4096)))
+        assert int(got[1]) == int(a.min()) and int(got[2]) == int(a.max())
+    ref = float(((x - x.mean()) ** 2).sum())
+    assert abs(raw[3] - ref) <= 1e-13 * ref + 1e-300
