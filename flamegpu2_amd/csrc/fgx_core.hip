@@ -93,13 +93,6 @@ __global__ void k_set_counts(SetCounts a) {
     if (t == 63 && a.inc) *a.inc += 1u;
 }
 
-__global__ void k_sub_u32(uint32_t* dst, const uint32_t* a, const uint32_t* b) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const uint32_t x = *a, y = *b;
-        *dst = x > y ? x - y : 0u;
-    }
-}
-
 __global__ void k_add_u32_n(uint32_t* __restrict__ p, uint32_t n, uint32_t delta) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] += delta;
@@ -606,13 +599,6 @@ int fgx_layer_space_info(fgx_ctx* ctx, uint32_t* images, size_t* bytes) {
     if (!ctx) return fail(FGX_ERR_ARG, "fgx_layer_space_info: NULL context");
     if (images) *images = (uint32_t)ctx->c.layers.images.size();
     if (bytes) *bytes = ctx->c.layers.used;
-    return FGX_OK;
-}
-
-int fgx_sub_u32(uint32_t* dst, const uint32_t* a, const uint32_t* b, void* stream) {
-    if (!dst || !a || !b) return fail(FGX_ERR_ARG, "fgx_sub_u32: NULL pointer");
-    hipLaunchKernelGGL(k_sub_u32, dim3(1), dim3(64), 0, (hipStream_t)stream, dst, a, b);
-    FGX_HIP(hipGetLastError());
     return FGX_OK;
 }
 

@@ -1777,7 +1777,7 @@ inline void CUDASimulation::launch_function(detail::FnRT& f, void* st) {
 }
 
 // Launch record and grid of one agent function; the device-side preparation (new-agent
-// defaults, the launch count) is enqueued on `st`.
+// defaults) is enqueued on `st`.
 inline uint32_t CUDASimulation::prepare_function(detail::FnRT& f, void* st, detail::FnArgs& a) {
     auto& l = f.agent->states.at(f.in_state);
     if (f.cap < l.cap)

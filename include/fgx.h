@@ -326,8 +326,6 @@ int fgx_compact_prefix(fgx_ctx* ctx, const uint32_t* flags, uint32_t keep, const
 int fgx_append_range(fgx_ctx* ctx, const uint32_t* d_src_off, const uint32_t* d_n, uint32_t n_cap, uint32_t nvars,
                      const void* const* src, void* const* dst, const uint32_t* var_bytes, uint32_t* d_dst_count,
                      uint32_t dst_capacity, uint32_t* d_overflow, void* scratch, size_t scratch_bytes, void* stream);
-/* *dst = max(*a - *b, 0) on the device (enabled-agent counts). */
-int fgx_sub_u32(uint32_t* dst, const uint32_t* a, const uint32_t* b, void* stream);
 
 /* ---------------------------------------------------------------- scan
  * Exclusive prefix sum of n u32 (cub::DeviceScan::ExclusiveSum call sites,
