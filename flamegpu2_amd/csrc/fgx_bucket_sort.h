@@ -13,6 +13,8 @@ struct BucketPlan {
     uint32_t shift;       // bucket = key >> shift
     uint32_t buckets;
     uint32_t tiles;
+    uint32_t piece_log;   // elements of a piece of an oversize bucket: 1 << piece_log
+    uint32_t rows;        // words of bin counts of such pieces
 };
 
 // Whether n_cap elements over `bins` keys (of which about `used` occur) take this sort, and

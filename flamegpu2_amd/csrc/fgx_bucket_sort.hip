@@ -27,9 +27,11 @@ struct BucketArgs {
     const uint32_t* d_n;
     uint32_t n_cap;
     uint32_t shift, buckets, tiles, tile, bins;   // tile: elements a tile
+    uint32_t piece_log;   // elements of a piece of an oversize bucket: 1 << piece_log, no fewer than a block sorts
     const float* x;
     const float* y;
     const float* z;
+    uint32_t* rows;       // [pieces of oversize buckets][1 << shift] elements of each bin, or NULL: none of more than one piece
     uint32_t* counts;     // [tiles][buckets] elements; after the prefix pass those of the tiles before
     uint32_t* totals;     // [buckets] elements
     uint32_t* starts;     // [buckets + 1] first element
@@ -49,7 +51,15 @@ __device__ __forceinline__ uint32_t key_of(const BucketArgs& a, uint32_t i) {
 template <uint32_t W>
 __device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* s_red, uint32_t* total) {
     const uint32_t w = threadIdx.x >> 6;
-    const uint32_t incl = wave_inclusive_u32(v);
+    // the opaque lane keeps the lanes' shuffle addresses from being shared between calls: held
+    // over a whole kernel they are spilled
+    uint32_t lane = lane_id(), incl = v;
+    asm volatile("" : "+v"(lane));
+#pragma unroll
+    for (uint32_t o = 1; o < 64; o <<= 1) {
+        const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((lane - o) << 2), (int)incl);
+        incl += lane >= o ? b : 0u;
+    }
     __syncthreads();   // s_red may still be read by the call before
     if (lane_id() == 63) s_red[w] = incl;
     __syncthreads();
@@ -138,6 +148,25 @@ __device__ __forceinline__ uint32_t filled_tiles(uint32_t n, uint32_t size) {
     return f ? f : 1u;
 }
 
+// A bucket of more than one piece of P = 1 << log elements (sort_piece) has a row of bin counts
+// for each piece: that of the piece with the bucket's element e.  A bucket of m > P elements
+// owns rows floor(2 first / P) on, ceil(m / P) <= floor(2 m / P) of them, so those of different
+// buckets are apart and n elements need at most floor(2 n / P) rows.
+__device__ __forceinline__ uint32_t piece_row(uint32_t first, uint32_t e, uint32_t log) { return (2u * first >> log) + (e >> log); }
+
+// Adds 1 to rows[word] for each lane that is `on`: lanes with the same word as the first one
+// left add together, four times over (few bins that hold much); the rest one by one.
+__device__ __forceinline__ void count_in_row(uint32_t* rows, uint32_t word, bool on) {
+    uint64_t left = __ballot(on);
+    for (uint32_t r = 0; r < 4 && left; ++r) {
+        const uint32_t lane = (uint32_t)__builtin_ctzll(left);
+        const uint64_t same = __ballot(on && word == (uint32_t)__builtin_amdgcn_readlane((int)word, (int)lane));
+        if (lane_id() == lane) atomicAdd(rows + word, (uint32_t)__builtin_popcountll(same));
+        left &= ~same;
+    }
+    if ((left >> lane_id()) & 1ull) atomicAdd(rows + word, 1u);
+}
+
 // ---------------------------------------------------------------- count
 template <uint32_t BT, uint32_t ITEMS>
 __global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
@@ -151,6 +180,13 @@ __global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
     if (t == 0) s_met = 0u;
     __syncthreads();
     const uint32_t base = tile * BT * ITEMS;
+    if (a.rows) {
+        // this tile's share of the rows that n elements can need, for the split to count in
+        const uint32_t words = (2u * n >> a.piece_log) << a.shift;
+        const uint64_t share = (uint64_t)(2u * BT * ITEMS) << a.shift;
+        const uint32_t w0 = (uint32_t)(tile * share >> a.piece_log), w1 = (uint32_t)((tile + 1u) * share >> a.piece_log);
+        for (uint32_t k = w0 + t; k < w1 && k < words; k += BT) a.rows[k] = 0u;
+    }
     if (base < n) {
         uint32_t k[ITEMS];
 #pragma unroll
@@ -237,6 +273,8 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
     __shared__ alignas(16) uint16_t s_rows[W * MAXB];
     __shared__ uint32_t s_start[MAXB];
     __shared__ uint32_t s_delta[MAXB];
+    __shared__ uint32_t s_big[MAXB];   // first element of a bucket of more than one piece, or kNoBlock
+    __shared__ uint32_t s_any;         // whether there is such a bucket
     __shared__ uint32_t s_key[T];
     __shared__ uint16_t s_loc[T];
     __shared__ uint32_t s_red[W];
@@ -263,6 +301,7 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
         key[c] = cnt ? key_of(a, base + (e < cnt ? e : 0u)) : 0u;
     }
     zero_rows<BT>(s_rows, W * nb);
+    if (t == 0) s_any = 0u;
     __syncthreads();
 #pragma unroll
     for (uint32_t c = 0; c < ITEMS; ++c)
@@ -280,6 +319,9 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
             if (j >= q || b0 + j >= nb) continue;
             s_delta[b0 + j] = run + offset_of[j] - s_start[b0 + j];
             if (tile == 0) a.starts[b0 + j] = run;
+            const bool big = a.rows && total_of[j] > 1u << a.piece_log;
+            s_big[b0 + j] = big ? run : kNoBlock;
+            if (big) s_any = 1u;
             run += total_of[j];
         }
         if (tile == 0 && t == 0) a.starts[nb] = total;
@@ -297,6 +339,7 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
     }
     __syncthreads();
     const uint32_t mask = (1u << a.shift) - 1u;
+    const bool any = s_any != 0u;
     uint32_t src[ITEMS], dst[ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < ITEMS; ++j) {
@@ -308,6 +351,10 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
             src[j] = base + s_loc[p];
             a.fine[dst[j]] = (uint16_t)(k & mask);
             a.idx[dst[j]] = src[j];
+            if (any) {
+                const uint32_t first = s_big[k >> a.shift];
+                count_in_row(a.rows, (piece_row(first, dst[j] - first, a.piece_log) << a.shift) + (k & mask), first != kNoBlock);
+            }
         }
     }
     if (!*a.stage) return;
@@ -330,13 +377,11 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
 }
 
 // ---------------------------------------------------------------- sort within a bucket
-// Writes output elements first + [0, m): place p takes input element s_src[p] (or in[first + p]
-// when s_src is NULL).  Two places and up to eight 4-byte variables per thread are loaded
-// before the first store.
-template <uint32_t BT>
-__device__ __forceinline__ void write_sorted(const VarTable& vt, const uint32_t* s_src, const uint32_t* in, uint32_t first,
-                                             uint32_t m) {
-    constexpr uint32_t P = 2, V = 8;
+// Copies m elements, the p-th from input element place.src(p) to output element place.dst(p).
+// Two of them and up to eight 4-byte variables per thread are loaded before the first store.
+template <uint32_t BT, uint32_t V, typename Place>
+__device__ __forceinline__ void write_elements(const VarTable& vt, uint32_t m, Place place) {
+    constexpr uint32_t P = 2;
     for (uint32_t p0 = threadIdx.x; p0 < m; p0 += P * BT) {
         uint32_t e[P];
         bool on[P];
@@ -344,7 +389,7 @@ __device__ __forceinline__ void write_sorted(const VarTable& vt, const uint32_t*
         for (uint32_t j = 0; j < P; ++j) {
             const uint32_t p = p0 + j * BT;
             on[j] = p < m;
-            e[j] = on[j] ? (s_src ? s_src[p] : in[first + p]) : 0u;
+            e[j] = on[j] ? place.src(p) : 0u;
         }
         uint32_t r[4][P] = {};
         for (uint32_t v0 = 0; v0 < vt.n; v0 += V) {
@@ -364,7 +409,7 @@ __device__ __forceinline__ void write_sorted(const VarTable& vt, const uint32_t*
                     uint32_t* out = reinterpret_cast<uint32_t*>(vt.out[v0 + k]);
 #pragma unroll
                     for (uint32_t j = 0; j < P; ++j)
-                        if (on[j]) out[first + p0 + j * BT] = x[k][j];
+                        if (on[j]) out[place.dst(p0 + j * BT)] = x[k][j];
                     // the record's words are variables just loaded (a second gather of four words
                     // cost as much as four variables: 29.1 against 23.5 us for 1 M messages)
 #pragma unroll
@@ -375,16 +420,31 @@ __device__ __forceinline__ void write_sorted(const VarTable& vt, const uint32_t*
                     }
                 } else {
                     for (uint32_t j = 0; j < P; ++j)
-                        if (on[j]) copy_var(vt, v0 + k, e[j], first + p0 + j * BT);
+                        if (on[j]) copy_var(vt, v0 + k, e[j], place.dst(p0 + j * BT));
                 }
             }
         }
         if (vt.rec) {
 #pragma unroll
             for (uint32_t j = 0; j < P; ++j)
-                if (on[j]) reinterpret_cast<uint4*>(vt.rec)[first + p0 + j * BT] = make_uint4(r[0][j], r[1][j], r[2][j], r[3][j]);
+                if (on[j]) reinterpret_cast<uint4*>(vt.rec)[place.dst(p0 + j * BT)] = make_uint4(r[0][j], r[1][j], r[2][j], r[3][j]);
         }
     }
+}
+
+// Output elements first + [0, m): place p takes input element s_src[p] (or in[first + p] when
+// s_src is NULL).
+struct SortedPlace {
+    const uint32_t* s_src;
+    const uint32_t* in;
+    uint32_t first;
+    __device__ __forceinline__ uint32_t src(uint32_t p) const { return s_src ? s_src[p] : in[first + p]; }
+    __device__ __forceinline__ uint32_t dst(uint32_t p) const { return first + p; }
+};
+template <uint32_t BT>
+__device__ __forceinline__ void write_sorted(const VarTable& vt, const uint32_t* s_src, const uint32_t* in, uint32_t first,
+                                             uint32_t m) {
+    write_elements<BT, 8>(vt, m, SortedPlace{s_src, in, first});
 }
 
 // The same for a bucket whose variables the split has moved to the output arrays already: place
@@ -443,14 +503,15 @@ __device__ __forceinline__ void permute_sorted(const VarTable& vt, const uint32_
     }
 }
 
-// LDS of one sorting block: the split's counters, and in the same words (before they are
-// counted) the bins of a selected part of an oversize bucket; the sources of each place.
+// LDS of one sorting block: the split's counters (in a piece of an oversize bucket, after them,
+// the output element of each place), the bins' first places, the source of each place.
 template <uint32_t BT, uint32_t MAXF, uint32_t S>
 struct SortLds {
     static constexpr uint32_t kCap = BT * S;   // S elements per thread
     static constexpr uint32_t kRowWords = (BT / 64u) * MAXF / 2u;
-    uint32_t rows[kRowWords > kCap / 2u ? kRowWords : kCap / 2u];
-    uint32_t start[MAXF + 1];
+    uint32_t rows[kRowWords > kCap ? kRowWords : kCap];
+    uint32_t start[MAXF];
+    uint32_t dest[MAXF];   // oversize buckets: where a piece's elements of each bin go
     uint32_t src[kCap];
     uint32_t red[BT / 64u];
     uint32_t lo, hi;
@@ -458,9 +519,9 @@ struct SortLds {
 
 // Elements (f[c], id[c]) of chunk c < cw of each wave, m in all, numbered (wave, chunk, lane):
 // s.src[place] = id in stable order by f, s.start[f] = first place.
-template <uint32_t BT, uint32_t MAXF, uint32_t S>
-__device__ __forceinline__ void sort_in_lds(SortLds<BT, MAXF, S>& s, uint32_t keys, const uint32_t (&f)[S],
-                                            const uint32_t (&id)[S], uint32_t cw, uint32_t m) {
+template <uint32_t BT, uint32_t MAXF, uint32_t S, uint32_t C>
+__device__ __forceinline__ void sort_in_lds(SortLds<BT, MAXF, S>& s, uint32_t keys, const uint32_t (&f)[C],
+                                            const uint32_t (&id)[C], uint32_t cw, uint32_t m) {
     constexpr uint32_t W = BT / 64u;
     const uint32_t w = threadIdx.x >> 6, lane = lane_id();
     uint16_t* rows = reinterpret_cast<uint16_t*>(s.rows);
@@ -468,13 +529,13 @@ __device__ __forceinline__ void sort_in_lds(SortLds<BT, MAXF, S>& s, uint32_t ke
     zero_rows<BT>(rows, W * stride);
     __syncthreads();
 #pragma unroll
-    for (uint32_t c = 0; c < S; ++c)
+    for (uint32_t c = 0; c < C; ++c)
         if (c < cw && (w * cw + c) * 64u + lane < m) split_count(rows, w * stride, f[c]);
     __syncthreads();
     split_scan<W>(rows, stride, keys, s.start, s.red);
     const uint32_t bits = key_bits(keys);
 #pragma unroll
-    for (uint32_t c = 0; c < S; ++c) {
+    for (uint32_t c = 0; c < C; ++c) {
         if (c >= cw) continue;
         const bool valid = (w * cw + c) * 64u + lane < m;
         const uint32_t p = split_place(rows, s.start, w * stride, f[c], valid, bits);
@@ -483,96 +544,89 @@ __device__ __forceinline__ void sort_in_lds(SortLds<BT, MAXF, S>& s, uint32_t ke
     __syncthreads();
 }
 
-// A bucket of more elements than its block holds is shared by several blocks: block `piece`
-// orders the bins that start within its window of kCap / 2 places.  The bucket's bins are
-// counted, the bins of the window selected in order into LDS, and sorted there; a bin that is
-// larger than LDS is already in order and is written as it comes.
+struct PiecePlace {
+    const uint32_t* s_src;
+    const uint32_t* s_dst;
+    __device__ __forceinline__ uint32_t src(uint32_t p) const { return s_src[p]; }
+    __device__ __forceinline__ uint32_t dst(uint32_t p) const { return s_dst[p]; }
+};
+
+// An oversize bucket of m elements is shared by blocks of one piece each: block `piece` places
+// elements [piece * P, ...) of the bucket's order, in rounds of half of what its LDS holds (fewer
+// registers: a block's worth at once spilled 45, also where no bucket is oversize).
+// The split has counted the bins of every piece (a.rows), so a block knows from the rows of
+// the pieces before where its elements of each bin go, and reads no elements but its own: the
+// cost stays near linear however the bins are filled.  1,048,576 messages of 28 bytes in no order
+// 142 us, with half of them in one bin 138, all of them 82; 250,007 of them 42, 52 and 50.
+// (Counting the bucket and selecting from it in every piece cost m^2 / 4,096 reads: 3,466 and
+// 6,462 us of 1 M, 2,024 and 3,826 of 250,007.)
 template <uint32_t BT, uint32_t MAXF, uint32_t S>
-__device__ __forceinline__ void sort_piece(const BucketArgs& a, const VarTable& vt, SortLds<BT, MAXF, S>& s, uint32_t bucket, uint32_t first,
-                           uint32_t m, uint32_t piece, uint32_t pieces) {
-    constexpr uint32_t W = BT / 64u, kCap = SortLds<BT, MAXF, S>::kCap, kWindow = kCap / 2u;
+__device__ __forceinline__ void sort_piece(const BucketArgs& a, const VarTable& vt, SortLds<BT, MAXF, S>& s, uint32_t bucket,
+                                           uint32_t first, uint32_t m, uint32_t piece) {
+    constexpr uint32_t W = BT / 64u, C = S / 2u, kRound = BT * C;
     const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
-    const uint32_t keys = 1u << a.shift;
-    for (uint32_t k = t; k < keys; k += BT) s.start[k] = 0u;
-    if (t == 0) {
-        s.lo = 0xFFFFFFFFu;
-        s.hi = 0u;
+    const uint32_t keys = 1u << a.shift, P = 1u << a.piece_log, pieces = (m + P - 1u) >> a.piece_log;
+    // s.start: the bucket's elements of each bin; s.dest: those of the pieces before
+    for (uint32_t k = t; k < keys; k += BT) s.start[k] = s.dest[k] = 0u;
+    if (pieces == 1u) {
+        __syncthreads();
+        for (uint32_t e = t; e < m; e += BT) atomicAdd(&s.start[a.fine[first + e]], 1u);
+        __syncthreads();
+    } else {
+        const uint32_t* rows = a.rows + ((size_t)piece_row(first, 0u, a.piece_log) << a.shift);
+        for (uint32_t k = t; k < keys; k += BT) {
+            uint32_t all = 0, before = 0;
+            for (uint32_t r0 = 0; r0 < pieces; r0 += 8u) {
+                uint32_t c[8];
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j) c[j] = r0 + j < pieces ? rows[(size_t)(r0 + j) * keys + k] : 0u;
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j) {
+                    all += c[j];
+                    before += r0 + j < piece ? c[j] : 0u;
+                }
+            }
+            s.start[k] = all;
+            s.dest[k] = before;
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (uint32_t e = t; e < m; e += BT) atomicAdd(&s.start[a.fine[first + e]], 1u);
-    __syncthreads();
+    // s.dest: where this piece's elements of each bin go
     {
         const uint32_t q = (keys + BT - 1u) / BT, k0 = t * q;
         uint32_t sum = 0, total;
         for (uint32_t j = 0; j < q && k0 + j < keys; ++j) sum += s.start[k0 + j];
-        uint32_t run = block_prefix<W>(sum, s.red, &total);
-        const uint32_t lo = piece * kWindow, hi = piece + 1u == pieces ? 0xFFFFFFFFu : lo + kWindow;
+        uint32_t run = first + block_prefix<W>(sum, s.red, &total);
         for (uint32_t j = 0; j < q && k0 + j < keys; ++j) {
-            const uint32_t k = k0 + j, c = s.start[k];
-            s.start[k] = run;
-            if (run >= lo && run < hi) {
-                atomicMin(&s.lo, k);
-                if (c) atomicMax(&s.hi, k + 1u);
-                const uint32_t bin = (bucket << a.shift) + k;
-                if (a.start_out && bin < a.bins) a.start_out[bin] = first + run;
-            }
-            run += c;
+            const uint32_t bin = (bucket << a.shift) + k0 + j;
+            if (a.start_out && piece == 0 && bin < a.bins) a.start_out[bin] = run;
+            s.dest[k0 + j] += run;
+            run += s.start[k0 + j];
         }
-        if (t == 0) s.start[keys] = m;
     }
-    __syncthreads();
-    const uint32_t ka = s.lo, kb = s.hi;     // bins [ka, kb) hold the window's elements
-    if (ka >= kb) return;
-    const uint32_t p0 = s.start[ka], p1 = s.start[kb];
-    uint32_t kc = kb;                        // bins [ka, kc) are sorted in LDS
-    if (p1 - p0 > kCap) kc = kb - 1u;        // the last one is too large (all before it start within the window)
-    const uint32_t pc = s.start[kc];
-    __syncthreads();
-    uint32_t taken = 0, passed = 0;
-    uint16_t* s_fine = reinterpret_cast<uint16_t*>(s.rows);
-    for (uint32_t e0 = 0; e0 < m; e0 += BT) {
-        const uint32_t e = e0 + t;
-        const uint32_t f = e < m ? a.fine[first + e] : 0xFFFFFFFFu;
-        const bool sel = f >= ka && f < kc, big = f >= kc && f < kb;
-        const uint64_t ms = __ballot(sel), mb = __ballot(big);
-        __syncthreads();
-        if (lane == 0) s.red[w] = (uint32_t)__builtin_popcountll(ms) | (uint32_t)__builtin_popcountll(mb) << 16;
-        __syncthreads();
-        uint32_t before = 0, all = 0;
+    const uint32_t end = (piece + 1u) * P < m ? (piece + 1u) * P : m;
+    for (uint32_t e0 = piece * P; e0 < end; e0 += kRound) {
+        const uint32_t len = end - e0 < kRound ? end - e0 : kRound;
+        const uint32_t cw = ((len + 63u) / 64u + W - 1u) / W;
+        __syncthreads();   // the round before reads s.start, and moves s.dest on
+        uint32_t f[C], id[C];
 #pragma unroll
-        for (uint32_t k = 0; k < W; ++k) {
-            before += k < w ? s.red[k] : 0u;
-            all += s.red[k];
+        for (uint32_t c = 0; c < C; ++c) {
+            const uint32_t e = (w * cw + c) * 64u + lane;
+            f[c] = c < cw && e < len ? a.fine[first + e0 + e] : 0u;
+            id[c] = f[c] << 16 | e;   // a round is at most 2^16
         }
-        const uint64_t below = (1ull << lane) - 1ull;
-        if (sel) {
-            const uint32_t p = taken + (before & 0xFFFFu) + (uint32_t)__builtin_popcountll(ms & below);
-            s_fine[p] = (uint16_t)(f - ka);
-            s.src[p] = a.idx[first + e];
+        sort_in_lds(s, keys, f, id, cw, len);
+        // the split's counters are done with: the words hold each place's output element now
+        for (uint32_t p = t; p < len; p += BT) {
+            const uint32_t v = s.src[p], k = v >> 16;
+            s.rows[p] = s.dest[k] + (p - s.start[k]);
+            s.src[p] = a.idx[first + e0 + (v & 0xFFFFu)];
         }
-        if (big) {
-            const uint32_t p = first + pc + passed + (before >> 16) + (uint32_t)__builtin_popcountll(mb & below);
-            const uint32_t i = a.idx[first + e];
-            copy_element(vt, i, p);
-            write_record(vt, i, p);
-        }
-        taken += all & 0xFFFFu;
-        passed += all >> 16;
+        write_elements<BT, 4>(vt, len, PiecePlace{s.src, s.rows});   // a thread takes the places it has just written
+        __syncthreads();
+        for (uint32_t k = t; k < keys; k += BT) s.dest[k] += (k + 1u < keys ? s.start[k + 1u] : len) - s.start[k];
     }
-    __syncthreads();
-    if (!taken) return;
-    const uint32_t cw = ((taken + 63u) / 64u + W - 1u) / W;
-    uint32_t f[S], id[S];
-#pragma unroll
-    for (uint32_t c = 0; c < S; ++c) {
-        const uint32_t e = (w * cw + c) * 64u + lane;
-        const bool valid = c < cw && e < taken;
-        f[c] = valid ? s_fine[e] : 0u;
-        id[c] = valid ? s.src[e] : 0u;
-    }
-    __syncthreads();
-    sort_in_lds<BT, MAXF, S>(s, kc - ka, f, id, cw, taken);
-    write_sorted<BT>(vt, s.src, nullptr, first + p0, taken);
 }
 
 // Two blocks of 1,024 threads share a CU where S is 8 (at most 64 VGPRs): one loads while the
@@ -590,17 +644,18 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
     } else {
         // further blocks: the pieces after the first of buckets that one block does not hold
         const uint32_t q = (nb + BT - 1u) / BT, b0 = t * q, want = blockIdx.x - nb;
+        const uint32_t size = a.shift ? 1u << a.piece_log : kWindow;
         if (t == 0) s.lo = 0xFFFFFFFFu;
         uint32_t sum = 0, total;
         for (uint32_t j = 0; j < q && b0 + j < nb; ++j) {
             const uint32_t m = a.starts[b0 + j + 1u] - a.starts[b0 + j];
-            sum += m > kCap ? (m - 1u) / kWindow : 0u;
+            sum += m > kCap ? (m - 1u) / size : 0u;
         }
         uint32_t run = block_prefix<W>(sum, s.red, &total);
         if (want >= total) return;
         for (uint32_t j = 0; j < q && b0 + j < nb; ++j) {
             const uint32_t m = a.starts[b0 + j + 1u] - a.starts[b0 + j];
-            const uint32_t more = m > kCap ? (m - 1u) / kWindow : 0u;
+            const uint32_t more = m > kCap ? (m - 1u) / size : 0u;
             if (want >= run && want < run + more) {
                 s.lo = b0 + j;
                 s.hi = want - run + 1u;
@@ -615,7 +670,7 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
     const uint32_t first = a.starts[b], m = a.starts[b + 1u] - first;
     if (a.start_out && b == nb - 1u && piece == 0 && t == 0) a.start_out[a.bins] = first + m;
     if (a.shift == 0) {
-        // a bucket is one bin and already in order
+        // a bucket is one bin and already in order: pieces of kWindow elements
         if (a.start_out && piece == 0 && t == 0) a.start_out[b] = first;
         const uint32_t p = m > kCap ? piece * kWindow : 0u;
         const uint32_t len = m > kCap ? (m - p < kWindow ? m - p : kWindow) : m;
@@ -629,7 +684,7 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
         return;
     }
     if (m > kCap) {
-        sort_piece<BT, MAXF, S>(a, vt, s, b, first, m, piece, (m - 1u) / kWindow + 1u);
+        sort_piece<BT, MAXF, S>(a, vt, s, b, first, m, piece);
         return;
     }
     const bool staged = *a.stage != 0u;
@@ -643,7 +698,7 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
         id[c] = staged ? e : (valid ? a.idx[first + e] : 0u);
     }
     const uint32_t keys = 1u << a.shift;
-    sort_in_lds<BT, MAXF, S>(s, keys, f, id, cw, m);
+    sort_in_lds(s, keys, f, id, cw, m);
     if (a.start_out)
         for (uint32_t k = t; k < keys; k += BT)
             if ((b << a.shift) + k < a.bins) a.start_out[(b << a.shift) + k] = first + s.start[k];
@@ -667,7 +722,7 @@ __global__ void __launch_bounds__(BT) k_sort_one_block(BucketArgs a, VarTable vt
         f[c] = valid ? key_of(a, e) : 0u;
         id[c] = e;
     }
-    sort_in_lds<BT, MAXF, S>(s, a.bins, f, id, cw, n);
+    sort_in_lds(s, a.bins, f, id, cw, n);
     if (a.start_out) {
         for (uint32_t k = t; k < a.bins; k += BT) a.start_out[k] = s.start[k];
         if (t == 0) a.start_out[a.bins] = n;
@@ -723,8 +778,15 @@ bool bucket_plan(uint32_t n_cap, uint32_t bins, uint64_t used, BucketPlan* p) {
     p->tiles = ceil_div(n_cap, p->threads * p->items);
     // the tables fit the scratch that every bin sort of this size has
     if ((uint64_t)p->tiles * p->buckets > n_cap) return false;
-    if ((uint64_t)p->tiles + 2ull * p->buckets + 8ull > n_cap / 2) return false;
-    return true;
+    const uint64_t tables = (uint64_t)p->tiles + 2ull * p->buckets + 8ull;
+    // Pieces of oversize buckets hold what a block does (2,048, 8,192 or 16,384 elements); blocks
+    // of 256 threads take up to 8,192, round by round, where the rows of bin counts would not fit.
+    const uint32_t cap = p->threads * (p->items == 8 ? 16u : 8u);
+    for (p->piece_log = cap == 2048u ? 11u : (cap == 8192u ? 13u : 14u); ; ++p->piece_log) {
+        p->rows = p->shift && n_cap > 1u << p->piece_log ? (2u * n_cap >> p->piece_log) << p->shift : 0u;
+        if (tables + p->rows <= n_cap / 2) return true;
+        if (p->piece_log >= 13u) return false;
+    }
 }
 
 template <uint32_t BT, uint32_t ITEMS, uint32_t MAXB, uint32_t S>
@@ -736,8 +798,9 @@ static int launch_passes(const BucketArgs& a, const VarTable& vt, hipStream_t st
     FGX_HIP(hipGetLastError());
     hipLaunchKernelGGL((k_bucket_split<BT, ITEMS, MAXB>), dim3(a.tiles), dim3(BT), 0, st, a, vt);
     FGX_HIP(hipGetLastError());
-    // a bucket of m elements has (m - 1) / kWindow pieces after its first
-    hipLaunchKernelGGL((k_bucket_sort<BT, kMaxBins, S>), dim3(a.buckets + a.n_cap / kWindow), dim3(BT), 0, st, a, vt);
+    // a bucket of m elements has (m - 1) / size pieces after its first
+    const uint32_t size = a.shift ? 1u << a.piece_log : kWindow;
+    hipLaunchKernelGGL((k_bucket_sort<BT, kMaxBins, S>), dim3(a.buckets + a.n_cap / size), dim3(BT), 0, st, a, vt);
     FGX_HIP(hipGetLastError());
     return FGX_OK;
 }
@@ -754,6 +817,7 @@ int bucket_sort(const BucketPlan& p, const KeyArgs& ka, uint32_t bins, const uin
     a.tiles = p.tiles;
     a.tile = p.threads * p.items;
     a.bins = bins;
+    a.piece_log = p.piece_log;
     a.x = x;
     a.y = y;
     a.z = z;
@@ -770,6 +834,7 @@ int bucket_sort(const BucketPlan& p, const KeyArgs& ka, uint32_t bins, const uin
     a.totals = tables + 4;
     a.starts = a.totals + p.buckets;
     a.met = a.starts + p.buckets + 1;
+    if (p.rows) a.rows = a.met + p.tiles;
     a.idx = words_b;
     a.counts = words_c;
     // Elements of a tile that share a bucket lie next to each other in it; below 16 of them

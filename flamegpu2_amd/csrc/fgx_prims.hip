@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(kBlock) k_index_scatter(const uint32_t* d_n, u
 //   * beyond: a bitmap over a window of kMapWords * 32 input indices is set in LDS, and a
 //     member's rank is the number of set bits below its own (per-8-word prefix counts
 //     plus at most 8 word popcounts), window by window over [min, max] of the bin.
-// Work per bin is O(n_b) per window, so a build costs O(n) however the bins are filled.
+// Work per bin is O(n_b) per window of indices, one block a bin.
 constexpr uint32_t kSmallBin = 32;
 constexpr uint32_t kLdsBin = 2 * kBlock;
 constexpr uint32_t kMapWords = 16384;

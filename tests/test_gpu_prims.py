@@ -772,6 +772,65 @@ def test_index_sizes_and_shapes(ctx, what, dims, n, axis, positions, use_dn):
     _index_case(ctx, what, dims, n, axis, positions, by, use_dn)
 
 
+def _one_bin(rng, n):
+    return [np.full(n, 0.77) for _ in range(3)]
+
+
+def _half(rng, n):
+    at = rng.uniform(0, 1, n) < 0.5
+    return [np.where(at, 0.37, rng.uniform(0, 1, n)) for _ in range(3)]
+
+
+def _few_bins(rng, n):
+    return [0.4 + 0.05 * rng.integers(0, 3, n) for _ in range(3)]
+
+
+# Buckets of more elements than a block sorts, shared piece by piece (of 8,192 elements, from
+# 3 M on 16,384): a piece and one element more or less, several such buckets, one, and lists
+# whose blocks hold less than a piece (256 threads, 2,048 elements).
+@pytest.mark.parametrize("what,dims,n,axis,positions,use_dn", [
+    ("messages", 3, 6000, 12, _one_bin, None), ("messages", 3, 8192, 12, _one_bin, None), ("messages", 3, 8193, 12, _one_bin, None),
+    ("agents", 3, 16384, 12, _one_bin, None), ("messages", 2, 16385, 40, _few_bins, 16384), ("agents", 2, 40001, 60, _half, None),
+    ("messages", 3, 100003, 30, _half, 99999), ("messages", 2, 262143, 200, _one_bin, None), ("bucket", 1, 262143, 5000, _half, None),
+    ("messages", 3, 262144, 40, _one_bin, 8193), ("agents", 3, 33 * 8192, 41, _few_bins, None), ("messages", 3, 1000003, 63, _half, None),
+    ("bucket", 1, 1000003, 20000, _one_bin, 999999), ("messages", 2, 3145728 + 5, 800, _one_bin, None),
+    ("agents", 2, 3200001, 800, _half, 3145729), ("messages", 2, 3300000, 800, _few_bins, 16385)])
+def test_index_skewed(ctx, what, dims, n, axis, positions, use_dn):
+    by = [4, 4, 8, 4, 2, 4, 4, 4, 12] if n < 300000 else [4, 8, 1]
+    _index_case(ctx, what, dims, n, axis, positions, by, use_dn)
+
+
+def _build_ms(ctx, order, n, g):
+    """Milliseconds of a message index build of n elements of 28 bytes over g^3 bins."""
+    import time
+    from flamegpu2_amd import fgx
+    P = [(p * g * 0.5).astype(np.float32) for p in order(np.random.default_rng(n), n)]
+    m = fgx.spatial_meta(3, [0.0] * 3, [g * 0.5] * 3, 0.5)
+    d_in = [dev(p) for p in P] + [empty(n, np.float32) for _ in range(4)]
+    d_out = [empty(n, np.float32) for _ in range(7)]
+    pbm, sb = empty(m.bins + 1, np.uint32), fgx.scratch_bytes(fgx.FGX_OP_SPATIAL_BUILD, n, m.bins)
+    s = scratch(sb)
+    vi, vo = [ptr(t) for t in d_in], [ptr(t) for t in d_out]
+    best = 1e9
+    for _ in range(6):
+        sync()
+        t0 = time.perf_counter()
+        for _ in range(4):
+            fgx.spatial_build(ctx, m, n, *vi[:3], vi, vo, [4] * 7, ptr(pbm), ptr(s), sb)
+        sync()
+        best = min(best, (time.perf_counter() - t0) / 4 * 1e3)
+    return best
+
+
+# An index costs about the same however its bins are filled: with half or all of the list in
+# one bin 0.6 to 1.2 times that of one in no order, as measured, and 5 times on a machine that
+# does other things too.  Costs that grow with the square of a bin were 25 to 90 times.
+@pytest.mark.parametrize("n,g", [(250007, 40), (1 << 20, 64)])
+@pytest.mark.parametrize("order", [_one_bin, _half])
+def test_index_cost_of_skew(ctx, order, n, g):
+    assert _build_ms(ctx, order, n, g) <= 5 * _build_ms(ctx, _uniform, n, g)
+
+
 # Lists filled in part: fewer tiles with elements than XCDs, whole tiles, one element more.
 @pytest.mark.parametrize("what,dims,n,axis,filled", [
     ("messages", 3, 100003, 30, 1024), ("agents", 3, 100003, 30, 7 * 1024), ("messages", 2, 100003, 60, 9 * 1024 + 1),
