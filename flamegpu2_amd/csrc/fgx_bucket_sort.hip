@@ -5,6 +5,9 @@
 //   split   per tile: (bin within the bucket, element index) to the bucket, stably
 //   sort    per bucket: stable order by bin in LDS, the bin starts, and every variable
 //
+// A list whose keys never fall from one element to the next (agents that stay in their bins) is
+// copied by the split, and the sort has only the bins that no element begins left to write.
+//
 // Ranks are taken in list order (per-wave counters, and the lanes of a wave that share a
 // key), so no pass depends on the order in which atomics land and none has to restore it.
 // Lists of one tile are sorted by one block in one launch.
@@ -12,8 +15,11 @@
 // What bounds it: from some 100,000 elements on, the gathers and stores of the last pass;
 // below, the launches, of which there are four (the sort through global atomics takes
 // seven).  1,048,576 messages of 28 bytes over 64^3 bins, in the order of the step before:
-// 69.3 us with atomics, 52.1 us this way; 8,388,593 of 20 bytes in no order: 2,069 and 528 us;
-// sort of 250,007 agents: 36.4 and 31.2 us.
+// 69.3 us with atomics, 52.6 us this way; 8,388,593 of 20 bytes in no order: 2,069 and 530 us;
+// sort of 250,007 agents: 36.4 and 31.8 us.  Lists in order, 28 bytes, with atomics (which find
+// them in order too), as any other list this way, and copied: 250,007 messages 24.7, 30.7 and
+// 22.0 us, 1 M 38.6, 49.9 and 34.6, 4 M over 80,000 bins 72.8, 155 and 67; the two passes that find
+// the order cost other lists up to 0.5 us.
 #include "fgx_bucket_sort.h"
 
 #include <algorithm>
@@ -21,6 +27,12 @@
 namespace fgx {
 
 constexpr uint32_t kMaxBuckets = 2048;     // per-wave 16-bit counters of a split: 64 KB for 16 waves
+
+// How the last pass gets at a bucket's variables: from the whole list; from the bucket's place in
+// the output arrays, where the split has moved them (see k_bucket_split); or, of a list whose
+// keys never fall from one element to the next, from that same place in the list.
+constexpr uint32_t kGather = 0u, kStage = 1u, kCopy = 2u;
+constexpr uint32_t kDisorder = 1u << 31;   // of a tile: some element has a smaller key than the one before
 
 struct BucketArgs {
     KeyArgs ka;
@@ -35,9 +47,10 @@ struct BucketArgs {
     uint32_t* counts;     // [tiles][buckets] elements; after the prefix pass those of the tiles before
     uint32_t* totals;     // [buckets] elements
     uint32_t* starts;     // [buckets + 1] first element
-    uint32_t* met;        // [tiles] buckets that occur in the tile
-    uint32_t* stage;      // one word: the split moves the variables too (see k_bucket_split)
-    uint32_t stage_above; // sum of `met` above which it does; 0: never
+    uint32_t* met;        // [tiles] buckets that occur in the tile, and kDisorder
+    uint32_t* edges;      // [tiles][2] first and last key; in the words of idx, which the split writes
+    uint32_t* mode;       // how the list moves (kGather, kStage, kCopy); its elements; whether rows are counted
+    uint32_t stage_above; // sum of `met` above which the split moves the variables; 0: never
     uint16_t* fine;       // bin within the bucket, in bucket order
     uint32_t* idx;        // element index, in bucket order
     uint32_t* start_out;  // bin starts, or NULL
@@ -170,14 +183,17 @@ __device__ __forceinline__ void count_in_row(uint32_t* rows, uint32_t word, bool
 // ---------------------------------------------------------------- count
 template <uint32_t BT, uint32_t ITEMS>
 __global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
+    constexpr uint32_t W = BT / 64u;
     __shared__ uint32_t s_hist[kMaxBuckets];
     __shared__ uint32_t s_met;
-    const uint32_t t = threadIdx.x;
+    __shared__ uint32_t s_first[W], s_last[W];   // first and last key of each wave
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
     const uint32_t n = load_count(a.d_n, a.n_cap);
     const uint32_t tile = xcd_filled_block(filled_tiles(n, BT * ITEMS));
     if (tile == kNoBlock) return;
     for (uint32_t b = t; b < a.buckets; b += BT) s_hist[b] = 0u;
     if (t == 0) s_met = 0u;
+    if (t == 0 && tile == 0) a.mode[2] = 0u;
     __syncthreads();
     const uint32_t base = tile * BT * ITEMS;
     if (a.rows) {
@@ -187,16 +203,31 @@ __global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
         const uint32_t w0 = (uint32_t)(tile * share >> a.piece_log), w1 = (uint32_t)((tile + 1u) * share >> a.piece_log);
         for (uint32_t k = w0 + t; k < w1 && k < words; k += BT) a.rows[k] = 0u;
     }
+    // elements are numbered (wave, item, lane), so that nearly each one's predecessor is in its wave
     if (base < n) {
+        const uint32_t e0 = base + w * ITEMS * 64u + lane;
         uint32_t k[ITEMS];
 #pragma unroll
-        for (uint32_t j = 0; j < ITEMS; ++j) {
-            const uint32_t i = base + j * BT + t;
-            k[j] = key_of(a, i < n ? i : base) >> a.shift;
-        }
+        for (uint32_t j = 0; j < ITEMS; ++j) k[j] = key_of(a, e0 + j * 64u < n ? e0 + j * 64u : base);
+        uint32_t before = 0u;
+        bool fell = false;
 #pragma unroll
-        for (uint32_t j = 0; j < ITEMS; ++j)
-            if (base + j * BT + t < n) atomicAdd(&s_hist[k[j]], 1u);
+        for (uint32_t j = 0; j < ITEMS; ++j) {
+            const bool on = e0 + j * 64u < n;
+            // the key of the lane before (wave_shr:1); lane 0 keeps the item before's last
+            const uint32_t p = (uint32_t)__builtin_amdgcn_update_dpp((int)before, (int)k[j], 0x138, 0xF, 0xF, false);
+            const uint32_t b = k[j] >> a.shift;
+            fell = fell || (on && k[j] < p);
+            before = (uint32_t)__builtin_amdgcn_readlane((int)k[j], 63);
+            // lanes with the first one's bucket add together: most do in a list nearly in order
+            const bool with_first = b == __builtin_amdgcn_readfirstlane(b);
+            const uint64_t same = __ballot(on && with_first);
+            if (on && !with_first) atomicAdd(&s_hist[b], 1u);
+            if (lane == 0 && same) atomicAdd(&s_hist[b], (uint32_t)__builtin_popcountll(same));
+        }
+        if (lane == 0) s_first[w] = k[0];
+        if (lane == 0) s_last[w] = before;
+        if (__ballot(fell) && lane == 0) atomicOr(&s_met, kDisorder);
     }
     __syncthreads();
     uint32_t met = 0;
@@ -205,22 +236,49 @@ __global__ void __launch_bounds__(BT) k_bucket_count(BucketArgs a) {
         a.counts[(size_t)tile * a.buckets + b] = c;
         met += c ? 1u : 0u;
     }
-    if (!a.stage_above) return;
-    met = wave_sum_u32(met);
-    if (lane_id() == 0) atomicAdd(&s_met, met);
-    __syncthreads();
-    if (t == 0) a.met[tile] = s_met;
+    if (a.stage_above) {
+        met = wave_sum_u32(met);
+        if (lane == 0) atomicAdd(&s_met, met);
+        __syncthreads();
+    }
+    if (t < 64u) {
+        const bool fell = t && t < W && base + t * ITEMS * 64u < n && s_first[t] < s_last[t - 1u];
+        const uint32_t any = __ballot(fell) ? kDisorder : 0u;
+        if (t == 0) {
+            a.met[tile] = s_met | any;
+            a.edges[2u * tile] = s_first[0];
+            a.edges[2u * tile + 1u] = s_last[W - 1u];
+        }
+    }
 }
 
 // ---------------------------------------------------------------- prefix
 // Block g: buckets [64 g, 64 g + 64), one per lane; each of the 16 waves takes a run of the
-// tiles, 8 loads in flight.
+// tiles, 8 loads in flight.  One block more finds out how the list moves.
 __global__ void __launch_bounds__(1024) k_bucket_prefix(BucketArgs a) {
     __shared__ uint32_t s_sum[16][64];
     __shared__ uint32_t s_red[16];
+    __shared__ uint32_t s_fell;
     const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
     const uint32_t b = blockIdx.x * 64u + lane;
-    const uint32_t tiles = filled_tiles(load_count(a.d_n, a.n_cap), a.tile);
+    const uint32_t n = load_count(a.d_n, a.n_cap), tiles = filled_tiles(n, a.tile);
+    if (blockIdx.x * 64u >= a.buckets) {
+        uint32_t met = 0, fell = 0, all = 0;
+        if (threadIdx.x == 0) s_fell = 0u;
+        for (uint32_t t = threadIdx.x; t < tiles; t += 1024u) {
+            const uint32_t m = a.met[t];
+            met += m & ~kDisorder;
+            fell |= t && a.edges[2u * t] < a.edges[2u * t - 1u] ? kDisorder : m;
+        }
+        __syncthreads();
+        if (fell & kDisorder) s_fell = 1u;
+        block_prefix<16>(met, s_red, &all);
+        if (threadIdx.x == 0) {
+            a.mode[0] = !s_fell ? kCopy : (a.stage_above && all > a.stage_above ? kStage : kGather);
+            a.mode[1] = n;
+        }
+        return;
+    }
     const uint32_t per = (tiles + 15u) / 16u;
     const uint32_t t0 = w * per < tiles ? w * per : tiles, t1 = t0 + per < tiles ? t0 + per : tiles;
     const bool on = b < a.buckets;
@@ -250,14 +308,66 @@ __global__ void __launch_bounds__(1024) k_bucket_prefix(BucketArgs a) {
             run += c[j];
         }
     }
-    if (w == 0 && on) a.totals[b] = total;
-    if (blockIdx.x == 0) {
-        uint32_t met = 0, all = 0;
-        if (a.stage_above)
-            for (uint32_t t = threadIdx.x; t < tiles; t += 1024u) met += a.met[t];
-        block_prefix<16>(met, s_red, &all);
-        if (threadIdx.x == 0) *a.stage = a.stage_above && all > a.stage_above ? 1u : 0u;
+    if (w == 0 && on) {
+        a.totals[b] = total;
+        if (a.rows && total > 1u << a.piece_log) a.mode[2] = 1u;
     }
+}
+
+// ---------------------------------------------------------------- lists in order
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Elements [lo, hi) of every variable to the same places: 16 bytes a load, four variables in
+// flight.  lo is a multiple of 16, so the ranges start on 16 bytes where the arrays do.
+template <uint32_t BT>
+__device__ __forceinline__ void copy_range(const VarTable& vt, uint32_t lo, uint32_t hi) {
+    constexpr uint32_t V = 4;
+    const uint32_t t = threadIdx.x, even = lo + ((hi - lo) & ~15u);
+    for (uint32_t v0 = 0; v0 < vt.n; v0 += V) {
+        const u32x4* in[V];
+        u32x4* out[V];
+        uint32_t len[V], most = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < V; ++k) {
+            const uint32_t v = v0 + k < vt.n ? v0 + k : v0, b = vt.bytes[v];
+            const char* i = vt.in[v] + (size_t)lo * b;
+            char* o = vt.out[v] + (size_t)lo * b;
+            const bool aligned = (((uintptr_t)i | (uintptr_t)o) & 15u) == 0u;
+            in[k] = reinterpret_cast<const u32x4*>(i);
+            out[k] = reinterpret_cast<u32x4*>(o);
+            len[k] = aligned && v0 + k < vt.n ? (even - lo) / 16u * b : 0u;
+            most = len[k] > most ? len[k] : most;
+            if (!aligned && v0 + k < vt.n)
+                for (uint32_t e = lo + t; e < even; e += BT) copy_var(vt, v, e, e);
+        }
+        for (uint32_t c = t; c < most; c += BT) {
+            u32x4 x[V];
+#pragma unroll
+            for (uint32_t k = 0; k < V; ++k)
+                if (c < len[k]) x[k] = in[k][c];
+#pragma unroll
+            for (uint32_t k = 0; k < V; ++k)
+                if (c < len[k]) out[k][c] = x[k];
+        }
+    }
+    if (even + t < hi) copy_element(vt, even + t, even + t);   // the list's last few
+    for (uint32_t e = lo + t; e < hi; e += BT) write_record(vt, e, e);
+}
+
+// Elements [lo, hi) of a list in order, lo a multiple of 16: the copy, and the starts of the bins
+// of which they are the first, or of the empty bins before, as far as the element's bucket
+// goes (end_bucket writes the others).
+template <uint32_t BT>
+__device__ __forceinline__ void copy_in_order(const BucketArgs& a, const VarTable& vt, uint32_t lo, uint32_t hi) {
+    if (a.start_out) {
+        for (uint32_t e = lo + threadIdx.x; e < hi; e += BT) {
+            const uint32_t k = key_of(a, e), low = k >> a.shift << a.shift;
+            uint32_t p = __shfl_up(k, 1, 64);
+            if (lane_id() == 0 && e) p = key_of(a, e - 1u);
+            for (uint32_t j = e && p >= low ? p + 1u : low; j <= k; ++j) a.start_out[j] = e;
+        }
+    }
+    copy_range<BT>(vt, lo, hi);
 }
 
 // ---------------------------------------------------------------- split
@@ -273,13 +383,12 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
     __shared__ alignas(16) uint16_t s_rows[W * MAXB];
     __shared__ uint32_t s_start[MAXB];
     __shared__ uint32_t s_delta[MAXB];
-    __shared__ uint32_t s_big[MAXB];   // first element of a bucket of more than one piece, or kNoBlock
-    __shared__ uint32_t s_any;         // whether there is such a bucket
+    __shared__ uint32_t s_big[MAXB];   // if any: first element of a bucket of more than one piece, or kNoBlock
     __shared__ uint32_t s_key[T];
     __shared__ uint16_t s_loc[T];
     __shared__ uint32_t s_red[W];
     const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
-    const uint32_t n = load_count(a.d_n, a.n_cap), nb = a.buckets;
+    const uint32_t mode = a.mode[0], n = a.mode[1], any = a.mode[2], nb = a.buckets;
     const uint32_t tile = xcd_filled_block(filled_tiles(n, T));
     if (tile == kNoBlock) return;
     const uint32_t base = tile * T;
@@ -287,6 +396,19 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
     // this thread's buckets: their totals and the tile's offsets are loaded beside the positions
     constexpr uint32_t Q = MAXB / BT;
     const uint32_t q = (nb + BT - 1u) / BT, b0 = t * q;
+    if (mode == kCopy) {
+        copy_in_order<BT>(a, vt, base, base + cnt);
+        if (tile) return;
+        uint32_t sum = 0, total;
+        for (uint32_t j = 0; j < q && b0 + j < nb; ++j) sum += a.totals[b0 + j];
+        uint32_t run = block_prefix<W>(sum, s_red, &total);
+        for (uint32_t j = 0; j < q && b0 + j < nb; ++j) {
+            a.starts[b0 + j] = run;
+            run += a.totals[b0 + j];
+        }
+        if (t == 0) a.starts[nb] = total;
+        return;
+    }
     uint32_t total_of[Q], offset_of[Q];
 #pragma unroll
     for (uint32_t j = 0; j < Q; ++j) {
@@ -301,7 +423,6 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
         key[c] = cnt ? key_of(a, base + (e < cnt ? e : 0u)) : 0u;
     }
     zero_rows<BT>(s_rows, W * nb);
-    if (t == 0) s_any = 0u;
     __syncthreads();
 #pragma unroll
     for (uint32_t c = 0; c < ITEMS; ++c)
@@ -319,9 +440,6 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
             if (j >= q || b0 + j >= nb) continue;
             s_delta[b0 + j] = run + offset_of[j] - s_start[b0 + j];
             if (tile == 0) a.starts[b0 + j] = run;
-            const bool big = a.rows && total_of[j] > 1u << a.piece_log;
-            s_big[b0 + j] = big ? run : kNoBlock;
-            if (big) s_any = 1u;
             run += total_of[j];
         }
         if (tile == 0 && t == 0) a.starts[nb] = total;
@@ -339,7 +457,15 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
     }
     __syncthreads();
     const uint32_t mask = (1u << a.shift) - 1u;
-    const bool any = s_any != 0u;
+    if (any) {
+#pragma unroll
+        for (uint32_t j = 0; j < Q; ++j) {
+            if (j >= q || b0 + j >= nb) continue;
+            const uint32_t first = s_delta[b0 + j] + s_start[b0 + j] - offset_of[j];
+            s_big[b0 + j] = total_of[j] > 1u << a.piece_log ? first : kNoBlock;
+        }
+        __syncthreads();
+    }
     uint32_t src[ITEMS], dst[ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < ITEMS; ++j) {
@@ -357,7 +483,7 @@ __global__ void __launch_bounds__(BT) k_bucket_split(BucketArgs a, VarTable vt) 
             }
         }
     }
-    if (!*a.stage) return;
+    if (mode != kStage) return;
     for (uint32_t v = 0; v < vt.n; ++v) {
         if (vt.bytes[v] == 4) {
             const uint32_t* in = reinterpret_cast<const uint32_t*>(vt.in[v]);
@@ -552,7 +678,7 @@ struct PiecePlace {
 };
 
 // An oversize bucket of m elements is shared by blocks of one piece each: block `piece` places
-// elements [piece * P, ...) of the bucket's order, in rounds of half of what its LDS holds (fewer
+// elements [piece * P, ...) of the bucket's order, in rounds of a quarter of what its LDS holds (fewer
 // registers: a block's worth at once spilled 45, also where no bucket is oversize).
 // The split has counted the bins of every piece (a.rows), so a block knows from the rows of
 // the pieces before where its elements of each bin go, and reads no elements but its own: the
@@ -563,7 +689,7 @@ struct PiecePlace {
 template <uint32_t BT, uint32_t MAXF, uint32_t S>
 __device__ __forceinline__ void sort_piece(const BucketArgs& a, const VarTable& vt, SortLds<BT, MAXF, S>& s, uint32_t bucket,
                                            uint32_t first, uint32_t m, uint32_t piece) {
-    constexpr uint32_t W = BT / 64u, C = S / 2u, kRound = BT * C;
+    constexpr uint32_t W = BT / 64u, C = S / 4u, kRound = BT * C;
     const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id();
     const uint32_t keys = 1u << a.shift, P = 1u << a.piece_log, pieces = (m + P - 1u) >> a.piece_log;
     // s.start: the bucket's elements of each bin; s.dest: those of the pieces before
@@ -629,6 +755,17 @@ __device__ __forceinline__ void sort_piece(const BucketArgs& a, const VarTable& 
     }
 }
 
+// The bins after the last element of this block's bucket, of a list that is in order.
+template <uint32_t BT>
+__device__ __forceinline__ void end_bucket(const BucketArgs& a) {
+    const uint32_t b = blockIdx.x;
+    if (!a.start_out || b >= a.buckets) return;
+    const uint32_t first = a.starts[b], next = a.starts[b + 1u], b0 = b << a.shift;
+    const uint32_t end = a.bins - b0 < 1u << a.shift ? a.bins : b0 + (1u << a.shift);
+    for (uint32_t k = (next > first ? key_of(a, next - 1u) + 1u : b0) + threadIdx.x; k < end; k += BT) a.start_out[k] = next;
+    if (b == a.buckets - 1u && threadIdx.x == 0) a.start_out[a.bins] = next;
+}
+
 // Two blocks of 1,024 threads share a CU where S is 8 (at most 64 VGPRs): one loads while the
 // other ranks.
 template <uint32_t BT, uint32_t MAXF, uint32_t S>
@@ -636,12 +773,15 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
     constexpr uint32_t W = BT / 64u, kCap = SortLds<BT, MAXF, S>::kCap, kWindow = kCap / 2u;
     __shared__ SortLds<BT, MAXF, S> s;
     const uint32_t t = threadIdx.x, w = t >> 6, lane = lane_id(), nb = a.buckets;
-    uint32_t b, piece = 0;
-    if (blockIdx.x < nb) {
-        // one block per bucket, neighbouring buckets on one XCD
-        const uint32_t x = blockIdx.x % 8u, k = blockIdx.x / 8u, q = nb / 8u, r = nb % 8u;
-        b = x * q + (x < r ? x : r) + k;
-    } else {
+    // one block per bucket, neighbouring buckets on one XCD
+    uint32_t b = blockIdx.x < nb ? xcd_filled_block(nb) : 0u, piece = 0;
+    uint32_t first = a.starts[b], next = a.starts[b + 1u];
+    const uint32_t mode = *a.mode;
+    if (mode == kCopy) {
+        end_bucket<BT>(a);
+        return;
+    }
+    if (blockIdx.x >= nb) {
         // further blocks: the pieces after the first of buckets that one block does not hold
         const uint32_t q = (nb + BT - 1u) / BT, b0 = t * q, want = blockIdx.x - nb;
         const uint32_t size = a.shift ? 1u << a.piece_log : kWindow;
@@ -666,8 +806,10 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
         b = s.lo;
         piece = s.hi;
         __syncthreads();
+        first = a.starts[b];
+        next = a.starts[b + 1u];
     }
-    const uint32_t first = a.starts[b], m = a.starts[b + 1u] - first;
+    const uint32_t m = next - first;
     if (a.start_out && b == nb - 1u && piece == 0 && t == 0) a.start_out[a.bins] = first + m;
     if (a.shift == 0) {
         // a bucket is one bin and already in order: pieces of kWindow elements
@@ -687,7 +829,7 @@ __global__ void __launch_bounds__(BT, S == 8 ? 8 : 4) k_bucket_sort(BucketArgs a
         sort_piece<BT, MAXF, S>(a, vt, s, b, first, m, piece);
         return;
     }
-    const bool staged = *a.stage != 0u;
+    const bool staged = mode == kStage;
     const uint32_t cw = ((m + 63u) / 64u + W - 1u) / W;
     uint32_t f[S], id[S];
 #pragma unroll
@@ -794,7 +936,7 @@ static int launch_passes(const BucketArgs& a, const VarTable& vt, hipStream_t st
     constexpr uint32_t kWindow = BT * S / 2u;
     hipLaunchKernelGGL((k_bucket_count<BT, ITEMS>), dim3(a.tiles), dim3(BT), 0, st, a);
     FGX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_bucket_prefix, dim3(ceil_div(a.buckets, 64)), dim3(1024), 0, st, a);
+    hipLaunchKernelGGL(k_bucket_prefix, dim3(ceil_div(a.buckets, 64) + 1u), dim3(1024), 0, st, a);
     FGX_HIP(hipGetLastError());
     hipLaunchKernelGGL((k_bucket_split<BT, ITEMS, MAXB>), dim3(a.tiles), dim3(BT), 0, st, a, vt);
     FGX_HIP(hipGetLastError());
@@ -830,12 +972,12 @@ int bucket_sort(const BucketPlan& p, const KeyArgs& ka, uint32_t bins, const uin
     // words_a: n_cap 16-bit bins, then the small tables; words_b: indices; words_c: the counts
     a.fine = reinterpret_cast<uint16_t*>(words_a);
     uint32_t* tables = words_a + (n_cap + 1u) / 2u;
-    a.stage = tables;
+    a.mode = tables;
     a.totals = tables + 4;
     a.starts = a.totals + p.buckets;
     a.met = a.starts + p.buckets + 1;
     if (p.rows) a.rows = a.met + p.tiles;
-    a.idx = words_b;
+    a.idx = a.edges = words_b;
     a.counts = words_c;
     // Elements of a tile that share a bucket lie next to each other in it; below 16 of them
     // (a half cache line of a 4-byte variable) gathering from the whole list costs more than
