@@ -442,9 +442,12 @@ constexpr uint32_t kHashId = name_hash("id", 3);
 // takes the lowest remaining one whenever its current unit ends.
 //
 // Over large lists the walk is bound by vector issue (boids, 1 M: 211 M wave instructions,
-// 118 a candidate, 343 us): scalar bases with 32-bit lane offsets (load_msg_var, fetch),
-// virtual coordinates only where a search can wrap (near_origin) and a shorter unit step
-// (take_unit) leave 165 M (92 a candidate) and, with blocks of 1024, 290 us.
+// 118 a candidate, 343 us): scalar bases with 32-bit lane offsets (load_msg_var, fetch) and a
+// shorter unit step (take_unit) take it, with blocks of 1024, to %1M us.  Small launches (one wave
+// a SIMD) wait instead, about 1,500 cycles a candidate, and what takes a scalar branch there
+// costs them more than vector instructions: skipping the virtual coordinates of waves whose
+// searches cannot wrap saved 1 % of 1 M boids and cost 5 % of 131,072 and fewer (1,024
+// boids 106.9 against 101.7 us, 65,536 107.6 / 102.4, 1 M 277.0 / 279.6).
 //
 // Source: the message list in HBM (bin table pbm, packed records), or, in the staged
 // kernel when every lane of the wave is covered by the block's LDS copy, the LDS tables
@@ -481,10 +484,6 @@ class SpatialFilter {
         id_err_ = id_ok ? 0u : (id_known ? (uint32_t)detail::DERR_MSG_VAR_TYPE : (uint32_t)detail::DERR_UNKNOWN_MSG_VAR);
         pbm_ = m.pbm;
         rec_ = reinterpret_cast<const char*>(c.a.in_meta.packed);   // the launch's (a batch: all simulations')
-        if (WRAP) {
-            flat_ = __builtin_amdgcn_readfirstlane(
-                __all(flat(m, 0, cx) && flat(m, 1, cy) && (DIMS == 2 || flat(m, 2, cz))) ? 1 : 0);
-        }
         sv_ = nullptr;
         tab_ = nullptr;
         tm_ = 0u;
@@ -542,9 +541,9 @@ class SpatialFilter {
             return detail::load_elem<T>(f_.c_.a.msg_in, f_.c_.a.msg_in_mul, name, g_, L, e, f_.c_,
                                         detail::DERR_UNKNOWN_MSG_VAR, detail::DERR_MSG_VAR_TYPE);
         }
-        __device__ __forceinline__ float getVirtualX() const { return near_origin(0, x_); }
-        __device__ __forceinline__ float getVirtualY() const { return near_origin(1, y_); }
-        __device__ __forceinline__ float getVirtualZ() const { return near_origin(2, z_); }
+        __device__ __forceinline__ float getVirtualX() const { return getVirtualX(f_.loc_[0]); }
+        __device__ __forceinline__ float getVirtualY() const { return getVirtualY(f_.loc_[1]); }
+        __device__ __forceinline__ float getVirtualZ() const { return getVirtualZ(f_.loc_[2]); }
         __device__ __forceinline__ float getVirtualX(float x1) const { return detail::virtual_coord(x_, x1, f_.width_[0]); }
         __device__ __forceinline__ float getVirtualY(float y1) const { return detail::virtual_coord(y_, y1, f_.width_[1]); }
         __device__ __forceinline__ float getVirtualZ(float z1) const { return detail::virtual_coord(z_, z1, f_.width_[2]); }
@@ -552,15 +551,6 @@ class SpatialFilter {
 
      private:
         friend class iterator;
-        // virtual_coord towards the search origin.  On an axis along which the wave's searches
-        // cannot wrap it is the coordinate itself, and a scalar branch skips seven vector
-        // instructions (the empty asm keeps the compiler from computing both and selecting).
-        __device__ __forceinline__ float near_origin(int axis, float v) const {
-            if (WRAP && f_.flat_) return v;
-            float x = v;
-            asm volatile("" : "+v"(x));
-            return detail::virtual_coord(x, f_.loc_[axis], f_.width_[axis]);
-        }
         const SpatialFilter& f_;
         uint32_t g_;
         float x_, y_, z_;
@@ -682,16 +672,6 @@ class SpatialFilter {
     __device__ __forceinline__ iterator end() const { return iterator(*this); }
 
  private:
-    // 1 when virtual_coord leaves every candidate of the wave's searches as it is along axis k:
-    // no search reaches the first or last cell.  The messages it visits then lie in the cells
-    // their bins name (positions outside the grid, infinities and NaN are binned into the outer
-    // cells), less than span + 1 cells and a rounding from the origin, which is at most half the
-    // width: half a cell covers the rounding of floor((p - min) / cell) below 2^21 cells.
-    __device__ __forceinline__ bool flat(const detail::SpatialDev& m, int k, int cell) const {
-        const int R = m.span, g = (int)m.grid[k];
-        const bool reach = ((float)R + 1.5f) * m.cell <= 0.5f * m.width[k] && g < (1 << 21);
-        return reach && cell - R >= 1 && cell + R <= g - 2;
-    }
     // Per-lane search origin.  HBM: bins of the grid.  LDS (ebase/xbase/width of the
     // covering group): virtual bin entries, rows of `width` entries for the 9 (3)
     // neighbour rows, x counted from xbase.
@@ -991,7 +971,6 @@ class SpatialFilter {
     int ebase_, xbase_, ewidth_;    // LDS source: covering group
     const uint32_t* pbm_;
     const char* rec_;               // packed 16-byte {x, y, z, id} record per message (HBM source)
-    uint32_t flat_;                 // wrapping: 1 when no search of the wave wraps (wave-uniform)
     uint32_t id_err_;
 };
 
@@ -1622,8 +1601,10 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t blocks) {
 // runs over the blocks with agents: a list filled to 40 % would keep only 4 of the 8 XCDs busy
 // (predator-prey, 1 M prey and 250 k predators, lists about 40 % full: the layers' launches
 // 183 us on average that way, 110 so).  At least 1: block 0 writes the message count of an empty list.
-__device__ __forceinline__ uint32_t filled_blocks(uint32_t n) {
-    const uint32_t b = (__builtin_amdgcn_readfirstlane(n) + blockDim.x - 1u) / blockDim.x;
+// Blocks are of 256, 512 or 1,024 threads; a division by their size would be 40 instructions
+// between the count and the first load (3 us of the 1,024-boid kernel's 107).
+__device__ __forceinline__ uint32_t filled_blocks(uint32_t n, uint32_t size) {
+    const uint32_t b = (__builtin_amdgcn_readfirstlane(n) + size - 1u) >> __builtin_ctz(size);
     return b ? b : 1u;
 }
 
@@ -1656,14 +1637,21 @@ __device__ __forceinline__ __attribute__((address_space(3))) uint32_t* wave_tabl
 // device memory).
 template <typename F, bool WIDE = false>
 __device__ __forceinline__ void run_function_block(const FnArgs& a, uint32_t x, uint32_t k) {
-    const uint32_t first = a.d_first ? load_count(a.d_first) : 0u;
-    const uint32_t n = a.d_n ? load_count(a.d_n) : a.n_cap;
-    const uint32_t blk = xcd_block(x, k, filled_blocks(n > first ? n - first : 0u));
+    // the empty asm has these loaded at once, where each would wait for the one before
+    const uint32_t* d_first = a.d_first;
+    const uint32_t* d_n = a.d_n;
+    uint32_t* d_messages = a.d_msg_count_out;
+    uint32_t* d_launched = a.d_launch_count_out;
+    uint32_t size = blockDim.x;
+    asm volatile("" : "+s"(d_first), "+s"(d_n), "+s"(d_messages), "+s"(d_launched), "+s"(size));
+    const uint32_t first = d_first ? load_count(d_first) : 0u;
+    const uint32_t n = d_n ? load_count(d_n) : a.n_cap;
+    const uint32_t blk = xcd_block(x, k, filled_blocks(n > first ? n - first : 0u, size));
     if (blk == kNoBlock) return;
-    const uint32_t o = blk * blockDim.x + threadIdx.x;
+    const uint32_t o = blk * size + threadIdx.x;
     if (o == 0) {
-        if (a.d_msg_count_out) *a.d_msg_count_out = n;   // one message per agent (no condition here)
-        if (a.d_launch_count_out) *a.d_launch_count_out = n > first ? n - first : 0u;
+        if (d_messages) *d_messages = n;   // one message per agent (no condition here)
+        if (d_launched) *d_launched = n > first ? n - first : 0u;
     }
     if (first + o >= n) return;
     const uint32_t i = first + o;
@@ -2000,7 +1988,7 @@ __global__ void __launch_bounds__(256) agent_function_kernel_staged(const FnArgs
     extern __shared__ uint32_t fgx_stage_smem[];
     __shared__ StageHeader sh;
     const uint32_t n = a.d_n ? load_count(a.d_n) : a.n_cap;
-    const uint32_t blk = xcd_block(filled_blocks(n));
+    const uint32_t blk = xcd_block(filled_blocks(n, blockDim.x));
     if (blk == kNoBlock) return;
     const uint32_t b0 = blk * blockDim.x;
     if (b0 == 0 && threadIdx.x == 0) {
