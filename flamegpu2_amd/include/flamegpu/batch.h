@@ -1609,14 +1609,18 @@ inline uint32_t BatchSimulation::readPopulation(int h, const std::string& agent,
     }
     uint32_t n = 0, o = 0;
     const List& l = part(s, agent, &o, &n);
+    std::vector<const detail::VarBuf*> vars;   // names first, as CUDASimulation::readPopulation
     for (auto& d : dst) {
         const detail::VarBuf* b = nullptr;
         for (auto& v : l.vars)
             if (v.name == d.first) b = &v;
         if (!b) throw exception::InvalidAgentVar("BatchSimulation: agent '" + agent + "' has no variable '" + d.first + "'");
-        detail::fgx_check(fgx_memcpy_d2h(d.second, (const char*)b->cur + (size_t)o * b->bytes, (size_t)n * b->bytes, stream_),
-                          "population download");
+        vars.push_back(b);
     }
+    for (size_t k = 0; k < dst.size(); ++k)
+        detail::fgx_check(fgx_memcpy_d2h(dst[k].second, (const char*)vars[k]->cur + (size_t)o * vars[k]->bytes,
+                                         (size_t)n * vars[k]->bytes, stream_),
+                          "population download");
     if (!dst.empty()) synchronize();
     return n;
 }

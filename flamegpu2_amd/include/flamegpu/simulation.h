@@ -1691,12 +1691,16 @@ inline uint32_t CUDASimulation::readPopulation(const std::string& agent, const s
     sync_counts();
     auto& l = it->second;
     check_device_error();
+    // names first: no copy into the caller's arrays is under way when an unknown one throws
+    std::vector<const detail::VarBuf*> vars;
     for (auto& d : dst) {
         const int vi = l.var_index(d.first);
         if (vi < 0) throw exception::InvalidAgentVar("Agent '" + a.d->name + "' does not contain variable '" + d.first + "'");
-        detail::fgx_check(fgx_memcpy_d2h(d.second, l.vars[vi].cur, (size_t)l.h_count * l.vars[vi].bytes, stream_),
-                          "population download");
+        vars.push_back(&l.vars[vi]);
     }
+    for (size_t k = 0; k < dst.size(); ++k)
+        detail::fgx_check(fgx_memcpy_d2h(dst[k].second, vars[k]->cur, (size_t)l.h_count * vars[k]->bytes, stream_),
+                          "population download");
     synchronize();
     return l.h_count;
 }
