@@ -443,7 +443,7 @@ constexpr uint32_t kHashId = name_hash("id", 3);
 //
 // Over large lists the walk is bound by vector issue (boids, 1 M: 211 M wave instructions,
 // 118 a candidate, 343 us): scalar bases with 32-bit lane offsets (load_msg_var, fetch) and a
-// shorter unit step (take_unit) take it, with blocks of 1024, to %1M us.  Small launches (one wave
+// shorter unit step (take_unit) take it, with blocks of 1024, to 281 us.  Small launches (one wave
 // a SIMD) wait instead, about 1,500 cycles a candidate, and what takes a scalar branch there
 // costs them more than vector instructions: skipping the virtual coordinates of waves whose
 // searches cannot wrap saved 1 % of 1 M boids and cost 5 % of 131,072 and fewer (1,024

@@ -1911,7 +1911,9 @@ inline bool CUDASimulation::launch_layer_fused(const LayerData& layer) {
     // The blocks start in the order of the functions here (the functions are independent): first
     // those that read the longer message lists, whose agents take longer, so that the launch
     // does not end on them with the chip half empty (predator-prey, 1 M prey fleeing 250 k predators and hunted
-    // by them in one layer: 335 us with the prey first, 257 us with the predators first).
+    // by them in one layer: 335 us with the prey first, 257 us with the predators first).  The
+    // list's capacity stands for the time of an agent, which also depends on how many messages
+    // lie near it: measured on this model only, and results do not depend on the order.
     std::vector<size_t> order(fl.size());
     for (size_t k = 0; k < fl.size(); ++k) order[k] = k;
     auto read = [&](size_t k) { return fl[k]->min ? fl[k]->min->cap : 0u; };
@@ -2135,10 +2137,13 @@ inline void CUDASimulation::enqueue_layer(const LayerData& layer) {
     }
     // auto spatial sort (CUDASimulation.cu:671-682) and lazy index builds.  Sorts move agent
     // lists and builds move message lists, so with in-layer concurrency on the builds of long
-    // lists run on a stream of their own beside the sorts.  The fork and the join take 18 us, more
-    // than the chains of short lists save (20 steps: predator-prey with 20 k prey 9.7 ms side by
-    // side, 9.0 in turn; 65,536 boids 3.59 / 3.53; 131,072 circles the same; 262,144 boids
-    // 4.33 / 4.41; predator-prey with 1 M prey, 10 steps, 9.6 / 10.0).
+    // lists run on a stream of their own beside the sorts.  The fork and the join take 10 to 18 us,
+    // more than the chains of short lists save.  Us a step side by side / in turn, with step
+    // graphs: 1,024 boids 134.7 / 127.0, 20,000 147.8 / 147.0, 65,536 154.8 / 156.9, 131,072
+    // 163.6 / 172.6, 262,144 183.0 / 194.1; circles of 1,024 156.8 / 149.5, 131,072 209.5 / 216.7;
+    // predator-prey with 20 k prey 332.7 / 315.7, 500 k 423.2 / 451.2.  Without graphs 1,024 boids
+    // 140.4 / 127.0, 65,536 158.6 / 159.1, 262,144 186.3 / 191.6; predator-prey 348.8 / 340.8
+    // and 450.4 / 460.0.
     constexpr uint32_t kOverlapAgents = 1u << 17;
     bool sorts = false, builds = false;
     uint32_t longest = 0;
