@@ -877,7 +877,8 @@ constexpr uint32_t kOneBlockMax = 4096u;
 constexpr uint32_t kMaxBins = 1024u;       // bins of a bucket: a sorting block's counters
 
 bool bucket_plan(uint32_t n_cap, uint32_t bins, uint64_t used, BucketPlan* p) {
-    // beyond 12 M elements the buckets outgrow their blocks
+    // 12.58 M elements are where measuring stopped: 2,048 buckets of 16,384 places would hold an
+    // evenly filled list of twice that
     if (!n_cap || !bins || n_cap > (3u << 22)) return false;
     *p = BucketPlan{};
     // one block sorts a list of 1,024 elements in 7 us; the four passes take 23 us on one of

@@ -441,13 +441,14 @@ constexpr uint32_t kHashId = name_hash("id", 3);
 // On the wave's unit table a lane starts with a bit mask of its non-empty units and
 // takes the lowest remaining one whenever its current unit ends.
 //
-// Over large lists the walk is bound by vector issue (boids, 1 M: 211 M wave instructions,
-// 118 a candidate, 343 us): scalar bases with 32-bit lane offsets (load_msg_var, fetch) and a
-// shorter unit step (take_unit) take it, with blocks of 1024, to 281 us.  Small launches (one wave
-// a SIMD) wait instead, about 1,500 cycles a candidate, and what takes a scalar branch there
-// costs them more than vector instructions: skipping the virtual coordinates of waves whose
-// searches cannot wrap saved 1 % of 1 M boids and cost 5 % of 131,072 and fewer (1,024
-// boids 106.9 against 101.7 us, 65,536 107.6 / 102.4, 1 M 277.0 / 279.6).
+// Over large lists the walk is bound by the gathers' address processing (boids, 1 M: the
+// texture-address unit 67 % busy, 78 % in the busiest CU) and the waits on them: scalar bases
+// with 32-bit lane offsets (load_msg_var, fetch), a shorter unit step (take_unit) and, for a
+// shared L1, blocks of 1024 take it from 343 us to 281, and its vector instructions from 118 a
+// candidate to 108.  Fewer alone gain nothing more: skipping the virtual coordinates of waves
+// whose searches cannot wrap left 92 and the same time (277.0 us against 279.6).  Small launches
+// (one wave a SIMD) wait for latency, about 1,500 cycles a candidate, and the scalar branches
+// of that skip cost them 5 %: 1,024 boids 106.9 us against 101.7, 65,536 107.6 against 102.4.
 //
 // Source: the message list in HBM (bin table pbm, packed records), or, in the staged
 // kernel when every lane of the wave is covered by the block's LDS copy, the LDS tables
