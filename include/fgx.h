@@ -58,7 +58,7 @@ int fgx_device_info(fgx_ctx* ctx, int* cu_count, int* xcd_count, size_t* hbm_byt
  * calls.  The bin sorts then leave their histogram zeroed behind them, and a sort on a
  * buffer that fgx_scratch_clear zeroed, or that the last sort used with the same bin
  * count, skips the clearing launch.  Under stream capture a sort skips it only when an
- * earlier sort of the buffer had to clear (sorts through LDS need not) and every one used
+ * earlier sort of the buffer used the histogram (sorts through LDS do not) and every one used
  * the same bin count; a buffer whose graphs are replayed must then keep that one bin count
  * in later sorts too (call fgx_scratch_clear and capture again after changing it). */
 enum { FGX_OPT_KEEP_SCRATCH_ZERO = 1 };
